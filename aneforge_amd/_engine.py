@@ -22,6 +22,7 @@ reconstructed exactly as the reference's constexpr ops would and streamed as fp1
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -234,12 +235,23 @@ def pack_encoded(fmt, w, s, bias=None) -> Linear:
 _GEMM_FMTS = ("int8", "fp16")                    # formats the prefill GEMM reads as packed
 
 
+@functools.lru_cache(maxsize=4096)
+def gemm_plan(fmt: str, M: int, N: int, Kd: int):
+    """(take the split GEMM, its workspace bytes) for M rows of a packed [N, Kd] weight: a pure function
+    of the shape, so a prompt's launches do not ask the library again."""
+    return K.gemm_split_plan(fmt, M, N, Kd)
+
+
 def prefill_gemm(eng, lin: "Linear", x, y, residual=None, epi="f16"):
-    """The batched prefill's linear: afx_gemm on the packed weights (int8, fp16), or on the fp16
-    expansion of the others in the engine's weight scratch (Q4_0, blockwise).  Prefill is
-    compute-bound, so one expansion per matrix per prompt chunk costs little; for blockwise it
-    measured faster than scaling the codes inside the GEMM (40.7 vs 48.2 ms for the 2048-token
-    cfg3 prompt: the in-GEMM products lengthen its LDS-bound fragment path)."""
+    """The batched prefill's linear.  The split GEMM reads every packed format and cuts K over the
+    chip; it is taken where its plan is the faster (up to a few hundred rows, further for the 4-bit
+    formats).  Otherwise afx_gemm on the packed weights (int8, fp16), or on the fp16 expansion of the
+    others in the engine's weight scratch (for blockwise that measured faster than scaling the codes
+    inside the GEMM: 40.7 vs 48.2 ms for the 2048-token cfg3 prompt)."""
+    split, ws_bytes = gemm_plan(lin.fmt, x.shape[0], lin.N, lin.K)
+    if split:
+        return K.gemm_split(lin.fmt, lin.w, lin.scale, x, y, bias=lin.bias, residual=residual, epi=epi,
+                            ws=eng.gemm_scratch(ws_bytes) if ws_bytes else None)
     if lin.fmt in _GEMM_FMTS:
         return K.gemm(lin.fmt, lin.w, lin.scale, x, y=y, bias=lin.bias, residual=residual, epi=epi)
     w16 = eng.weight_scratch(lin.N * lin.K).view(lin.N, lin.K)
@@ -606,6 +618,13 @@ class DecodeEngine:
         if getattr(self, "_w16", None) is None or self._w16.numel() < n:
             self._w16 = torch.empty(n, dtype=torch.float16, device="cuda")
         return self._w16[:n]
+
+    def gemm_scratch(self, nbytes: int) -> torch.Tensor:
+        """An fp32 workspace of at least nbytes for the split GEMM's partials (reused by every linear in
+        stream order; a prompt's largest is a few MB per hundred rows)."""
+        if getattr(self, "_gws", None) is None or self._gws.numel() * 4 < nbytes:
+            self._gws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device="cuda")
+        return self._gws
 
     def _prefill_buffers(self, C: int) -> dict:
         if getattr(self, "_pf", None) is None or self._pf["x"].shape[0] < C:

@@ -81,6 +81,8 @@ SIGNATURES: dict[str, tuple] = {
     "afx_topk_mask": (_i, [_vp, _i, _i, _i, _vp, _vp]),
     # batched prefill
     "afx_gemm": (_i, [_i, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _i, _vp]),
+    "afx_gemm_split": (_i, [_i, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _ll, _vp]),
+    "afx_gemm_split_plan": (_i, [_i, _i, _i, _i, _llp]),
     "afx_qkv_split_rope": (_i, [_vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp, _i, _vp, _vp, _ll, _i, _vp]),
     "afx_prefill_attn": (_i, [_vp, _i, _vp, _vp, _ll, _i, _vp, _i, _i, _i, _i, _i, _i, _f, _vp]),
     "afx_moe_combine": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),

@@ -1,0 +1,212 @@
+// C-ABI entry points, plan and finishing sum of the split GEMM (kernel: afx_gemm_split.h).
+#include <math.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include "afx_gemm_split.h"
+
+namespace afx {
+
+constexpr int kSplitMaxS = 16;
+
+static long long split_row_bytes_of(int fmt, int K) { return fmt == FMT_F16 ? 2LL * K : fmt == FMT_I8 || fmt == FMT_BW ? K : K / 2; }
+static long long split_side_bytes_of(int fmt, int K) {
+  return fmt == FMT_Q4 || fmt == FMT_BW ? K / 32 * 2 : fmt == FMT_Q4K ? K / 256 * 20 : fmt == FMT_Q6K ? K / 32 * 12 : 0;
+}
+
+bool split_supported(int fmt, int N, int K) {
+  return fmt >= 0 && fmt <= 6 && N >= 16 && N % 16 == 0 && K >= kSK && K % (fmt == FMT_Q4K || fmt == FMT_Q6K ? 256 : kSK) == 0;
+}
+
+// Microseconds of one workgroup and K chunk by row tile (16 * mt rows) and features (32 * nw), measured on
+// MI355X with int8 weights at 4096 x 4096 and 22016 x 4096; `busy` with every CU taken, where the taller
+// tiles, one workgroup per CU, slow down.  dec: what decoding a format's 128 features adds (none for int8
+// codes, two fp32 steps per weight for the K-quants; fp16: twice the bytes).
+static float split_chunk_us(int fmt, int mt, int nw, bool busy) {
+  const int i = mt <= 4 ? mt - 1 : mt <= 6 ? 4 : 5;
+  static const float c4[6] = {0.35f, 0.45f, 0.53f, 0.62f, 0.74f, 0.97f};
+  static const float c8[6] = {0.0f, 0.0f, 0.0f, 1.01f, 1.24f, 1.53f};
+  static const float dec[7] = {0.0f, 0.05f, 0.25f, 0.2f, 0.15f, 0.45f, 0.3f};
+  const float slow = !busy ? 1.0f : mt == 8 ? 1.2f : nw == 8 ? 1.2f : 1.0f;
+  return nw == 8 ? (c8[i] + 2.0f * dec[fmt]) * slow : (c4[i] + dec[fmt]) * slow * (nw == 4 ? 1.0f : 0.7f);
+}
+static double weight_mb(int fmt, int N, int K) {
+  return (double)N * (split_row_bytes_of(fmt, K) + split_side_bytes_of(fmt, K)) * 1e-6;
+}
+
+// The tile and slice count with the least predicted time: rounds of workgroups over the CUs (two resident
+// per CU up to 192 rows x features of 32, so rounds need not be whole there) x chunks x the chunk time,
+// a round's fill and drain, half of the weight stream's 5 TB/s time (the other half overlaps), and a second launch and about 0.5 us
+// per MB of partials when K is sliced.  Predictions are within 15% of what the shapes above measure at
+// 16 to 2048 rows: 4096 x 4096 at 64, 128 and 300 rows takes 13.6, 15.9 and 25.2 us where the 128 x 128
+// tiles of afx_gemm take 42.4, 42.5 and 43.7.
+SplitPlan split_plan(int fmt, int M, int N, int K) {
+  static const int mts[6] = {1, 2, 3, 4, 6, 8};
+  const char* es = getenv("AFX_GEMM_SPLIT");       // "S", "S.nw" or "S.nw.mt": a fixed choice (tests, tuning), read per call
+  int fs = 0, fn = 0, fm = 0;
+  if (es) sscanf(es, "%d.%d.%d", &fs, &fn, &fm);
+  const int nk = K / kSK, t16 = (M + 15) / 16;
+  SplitPlan best = {};
+  best.us = 1e30f;
+  for (int im = 0; im < 6; ++im) {
+    const int mt = mts[im];
+    if (fm ? mt != fm : im > 0 && mts[im - 1] >= t16) continue;      // no tile taller than needed
+    for (int nw = 2; nw <= 8; nw *= 2) {
+      if (!split_built(fmt, mt, nw)) continue;
+      if (fn && nw != fn) continue;
+      SplitPlan p = {mt, nw, (t16 + mt - 1) / mt, (N + 32 * nw - 1) / (32 * nw), 1, 0.0f};
+      const double part = (double)p.tiles_m * p.tiles_n * mt * nw * 2048e-6;   // MB of one slice's partials
+      const bool two = mt <= 6 && nw <= 4 && fmt != FMT_F16;
+      for (int S = 1; S <= kSplitMaxS && S <= nk; ++S) {
+        if (fs ? S != (fs < nk ? fs : nk) : S > 1 && nk / S < 2) continue;
+        const double wgs = (double)p.tiles_m * p.tiles_n * S;
+        const double rounds = wgs <= 256 ? 1.0 : two ? wgs / 256 + 0.25 : ceil(wgs / 256);
+        // a tile's epilogue (its K groups meet, then the stores) grows with its registers
+        const double tail = 0.0016 * (mt * nw) * (mt * nw);
+        const double us = 4.5 + rounds * tail + (rounds - 1) * (two ? 1.0 : 2.5) +
+                          rounds * ((nk + S - 1) / S) * split_chunk_us(fmt, mt, nw, wgs > 200) +
+                          weight_mb(fmt, N, K) / 10.0 + (S > 1 ? 2.0 + 0.5 * S * part : 0.0);
+        if (us < best.us) {
+          best = p;
+          best.S = S;
+          best.us = (float)us;
+        }
+      }
+    }
+  }
+  return best;
+}
+// The same product on afx_gemm's 128 x 128 tiles: 0.6 us per 64-wide step with up to a tile per CU, 0.575 us
+// per step and tile of a CU beyond that, after an expansion to fp16 (6 TB/s; the codebook and
+// K-quant kernels 4 and 2) for formats it does not read.
+static float gemm_tile_us(int fmt, int M, int N, int K) {
+  const double tiles = (double)((M + 127) / 128) * ((N + 127) / 128);
+  double us = 4.5 + (K / 64) * (tiles <= 256 ? 0.6 : 0.575 * tiles / 256 + 0.15) + weight_mb(fmt, N, K) / 12.0;
+  if (fmt != FMT_I8 && fmt != FMT_F16) {
+    const double tbs = fmt == FMT_Q6K ? 2.0 : fmt == FMT_Q4K || fmt == FMT_L4 ? 4.0 : 6.0;
+    us += 2.0 + (2e-6 * N * K + weight_mb(fmt, N, K)) / tbs;
+  }
+  return (float)us;
+}
+static long long split_ws_bytes(const SplitPlan& p, int S) {
+  return (long long)S * p.tiles_m * p.tiles_n * p.mt * p.nw * 2048;
+}
+
+// y = epilogue(sum of the S slices of ws in slice order), four output features of one row per thread;
+// the slices hold the tiles in the kernel's own order.
+__global__ __launch_bounds__(256) void gemm_split_finish_kernel(SplitArgs a) {
+  const int nt = 2 * a.nw;
+  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long per = (long long)a.tiles_m * a.tiles_n * nt * a.mt * 64;   // f4 per slice
+  if (idx >= per) return;
+  const int lane = (int)(idx & 63), q0 = (int)(idx >> 6), q1 = q0 / a.mt, tile = q1 / nt;
+  const int n = (tile / a.tiles_m) * (16 * nt) + 16 * (q1 % nt) + 4 * (lane >> 4);
+  const int m = ((tile % a.tiles_m) * a.mt + q0 % a.mt) * 16 + (lane & 15);
+  if (n >= a.N || m >= a.M) return;
+  const f4* w = (const f4*)a.ws + idx;
+  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int q = 0; q < a.S; q += 4) {               // four slices' loads in flight; slots past S re-read the first
+    f4 t[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) t[u] = w[(q + u < a.S ? q + u : 0) * per];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (q + u < a.S) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += t[u][i];
+      }
+  }
+  split_store4(a, v, n, m);
+}
+
+static split_fn pick(int fmt, int mt, int nw) {
+  switch (fmt) {
+    case FMT_I8: return pick_split<FMT_I8>(mt, nw);
+    case FMT_Q4: return pick_split<FMT_Q4>(mt, nw);
+    case FMT_F16: return pick_split<FMT_F16>(mt, nw);
+    case FMT_BW: return pick_split<FMT_BW>(mt, nw);
+    case FMT_L4: return pick_split<FMT_L4>(mt, nw);
+    case FMT_Q4K: return pick_split<FMT_Q4K>(mt, nw);
+    default: return pick_split<FMT_Q6K>(mt, nw);
+  }
+}
+
+// Experts: the row tile covers about 1.25 times the mean tokens of an expert (a longer list takes several
+// tiles); the grid holds the most row tiles T * topk entries can make.
+int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what) {
+  AFX_REQUIRE(a.w && a.x && a.y && a.cnt && a.list, "%s: null pointer", what);
+  AFX_REQUIRE(a.T >= 1 && a.topk >= 1 && a.E >= 1 && split_supported(fmt, a.N, a.K), "%s: bad sizes", what);
+  AFX_REQUIRE(a.ldx % 8 == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.w & 15) == 0,
+              "%s: x and weights must be 16-byte aligned", what);
+  AFX_REQUIRE(fmt == FMT_F16 || a.scale, "%s: quantized weights need scales", what);
+  const long long entries = (long long)a.T * a.topk, xrows = a.x_by_token ? a.T : entries;
+  const long long xbytes = xrows * a.ldx * 2;
+  AFX_REQUIRE(xbytes < 0x7fff0000LL, "%s: activations span %lld bytes (limit 2 GiB)", what, xbytes);
+  a.xbytes = (int)xbytes;
+  const double mean = 1.25 * entries / a.E / 16;   // in 16-row tiles
+  const int mt = mean <= 1 ? 1 : mean <= 2 ? 2 : mean <= 3 ? 3 : mean <= 4 ? 4 : mean <= 6 ? 6 : 8;
+  const int nw = (double)((a.N + 127) / 128) * (a.E < entries ? a.E : entries) >= 256 ? 4 : 2;
+  a.S = 1; a.M = 0; a.mt = mt; a.nw = nw;
+  a.tiles_n = (a.N + 32 * nw - 1) / (32 * nw);
+  const long long tiles = entries / (16 * mt) + (a.E < entries ? a.E : entries);
+  AFX_REQUIRE(tiles * a.tiles_n < (1ll << 31), "%s: too many tiles", what);
+  const bool glu = a.epi == EPI_SWIGLU || a.epi == EPI_GEGLU;
+  a.vec = glu ? a.ldy % 2 == 0 && ((uintptr_t)a.y & 3) == 0 : a.ldy % 4 == 0 && ((uintptr_t)a.y & 15) == 0;
+  hipLaunchKernelGGL(pick(fmt, mt, nw), dim3((unsigned)(tiles * a.tiles_n)), dim3(512), 0, stream, a);
+  return check_launch(what);
+}
+
+}  // namespace afx
+
+using namespace afx;
+
+extern "C" {
+
+int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes) {
+  if (ws_bytes) *ws_bytes = 0;
+  AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K), "afx_gemm_split_plan: fmt=%d M=%d N=%d K=%d is not afx_gemm_split's", fmt, M, N, K);
+  const SplitPlan p = split_plan(fmt, M, N, K);
+  if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, p.S) : 0;
+  return p.us < 0.88f * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
+}
+
+int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int ldx, void* y, int ldy, int M, int N,
+                   int K, const void* bias, const void* residual, int epi, void* ws, long long ws_bytes,
+                   void* stream) {
+  AFX_REQUIRE(w && x && y, "afx_gemm_split: null pointer");
+  AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K),
+              "afx_gemm_split: need M >= 1, N %% 16 == 0, K %% 128 == 0 (256 for K-quants) (fmt=%d M=%d N=%d K=%d)", fmt, M, N, K);
+  AFX_REQUIRE(ldx >= K && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0,
+              "afx_gemm_split: x and weights must be 16-byte aligned rows (ldx %% 8 == 0)");
+  const long long xbytes = ((long long)(M - 1) * ldx + K) * 2;
+  AFX_REQUIRE(xbytes < (1ll << 31), "afx_gemm_split: activations span %lld bytes (limit 2 GiB)", xbytes);
+  AFX_REQUIRE((epi >= 0 && epi <= 3) || epi == EPI_GEGLU, "afx_gemm_split: unknown epilogue %d", epi);
+  AFX_REQUIRE(fmt == FMT_F16 || scale, "afx_gemm_split: quantized weights need scales");
+  const int align = fmt == FMT_L4 ? 15 : fmt == FMT_Q4 || fmt == FMT_BW ? 7 : fmt == FMT_Q4K || fmt == FMT_Q6K ? 3 : 1;
+  AFX_REQUIRE(((uintptr_t)scale & align) == 0, "afx_gemm_split: scales must be %d-byte aligned", align + 1);
+  AFX_REQUIRE(epi != EPI_RESID || residual, "afx_gemm_split: residual pointer required");
+  const bool glu = epi == EPI_SWIGLU || epi == EPI_GEGLU;
+  AFX_REQUIRE(glu ? ldy >= N / 2 : ldy >= N, "afx_gemm_split: ldy=%d too small", ldy);
+  AFX_REQUIRE(!ws || ((uintptr_t)ws & 15) == 0, "afx_gemm_split: the workspace must be 16-byte aligned");
+  SplitArgs a = {};
+  a.w = w; a.scale = (const half_t*)scale; a.bias = (const half_t*)bias; a.x = (const half_t*)x; a.y = y;
+  a.resid = (const half_t*)residual; a.ldx = ldx; a.ldy = ldy; a.M = M; a.N = N; a.K = K; a.epi = epi;
+  a.ws = (float*)ws;
+  a.xbytes = (int)xbytes;
+  const SplitPlan p = split_plan(fmt, M, N, K);
+  a.S = p.S;
+  while (a.S > 1 && (!ws || split_ws_bytes(p, a.S) > ws_bytes)) --a.S;
+  a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.mt = p.mt; a.nw = p.nw;
+  a.vec = epi == EPI_F32 ? ldy % 4 == 0 && ((uintptr_t)y & 15) == 0
+        : glu ? ldy % 2 == 0 && ((uintptr_t)y & 3) == 0
+        : ldy % 4 == 0 && ((uintptr_t)y & 7) == 0 && (epi != EPI_RESID || ((uintptr_t)residual & 7) == 0);
+  const long long blocks = ((long long)a.tiles_n * a.S + 7) / 8 * 8 * a.tiles_m;
+  AFX_REQUIRE(blocks < (1ll << 31), "afx_gemm_split: %lld tiles", blocks);
+  hipLaunchKernelGGL(pick(fmt, p.mt, p.nw), dim3((unsigned)blocks), dim3(512), 0, (hipStream_t)stream, a);
+  int rc = check_launch("afx_gemm_split");
+  if (rc || a.S == 1) return rc;
+  const long long n = split_ws_bytes(p, 1) / 16;
+  hipLaunchKernelGGL(gemm_split_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a);
+  return check_launch("afx_gemm_split(finish)");
+}
+
+}  // extern "C"

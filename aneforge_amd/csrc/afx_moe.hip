@@ -12,6 +12,7 @@
 // The grid covers all E experts; workgroups of experts with no tokens exit at once, so the
 // launch shape is fixed and the whole layer is graph-capturable (no host round trip).
 #include "afx_gemv_core.h"
+#include "afx_gemm_split.h"
 #include "afx_gemv_impl.h"
 #include "afx_mfma.h"
 
@@ -113,12 +114,12 @@ __device__ __forceinline__ void bucket_experts_wave(int s, int lane, int T, int 
 // experts l, l + 64, ..., l + 64 * (J - 1), J = ceil(E / 64) rounded up to an instantiated count.
 template <int J>
 __global__ __launch_bounds__(1024) void moe_topk_kernel(const float* __restrict__ logits, int T, int E, int k,
-                                                        int renorm, float* __restrict__ gate,
+                                                        int renorm, int many, float* __restrict__ gate,
                                                         int* __restrict__ sel, int* __restrict__ cnt,
                                                         int* __restrict__ list) {
-  extern __shared__ int s_sel[];   // [T][k]
+  extern __shared__ int s_sel[];   // [T][k] (unused when many)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int tt = wave; tt < T; tt += nw) {
+  for (int tt = blockIdx.x * nw + wave; tt < T; tt += nw * gridDim.x) {
     const float* lr = logits + (size_t)tt * E;
     float lg[J];
 #pragma unroll
@@ -132,11 +133,39 @@ __global__ __launch_bounds__(1024) void moe_topk_kernel(const float* __restrict_
     if (lane < k) {
       gate[(size_t)tt * k + lane] = g_r;
       sel[(size_t)tt * k + lane] = s_r;
-      s_sel[tt * k + lane] = s_r;
+      if (!many) s_sel[tt * k + lane] = s_r;
     }
   }
+  if (many) return;                                // moe_bucket_kernel makes the lists
   __syncthreads();
   bucket_experts(s_sel, T, E, k, cnt, list);
+}
+
+// The buckets of n = T * k selections with one wavefront per expert: 64 selections a pass, an entry's
+// place is the expert's count so far plus its earlier entries in the pass (token order, as
+// bucket_experts).  The one-workgroup form walks every selection in each expert's thread: 300 tokens
+// of top-2 took 63 us with it and the top-k in the same workgroup.
+__global__ __launch_bounds__(256) void moe_bucket_kernel(const int* __restrict__ sel, int T, int E, int k,
+                                                         int* __restrict__ cnt, int* __restrict__ list) {
+  const int lane = threadIdx.x & 63, e = blockIdx.x * 4 + (threadIdx.x >> 6), n = T * k;
+  if (e >= E) return;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int c = 0;
+  for (int i0 = 0; i0 < n; i0 += 64 * 4) {
+    int s[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + 64 * u + lane;
+      s[u] = i < n ? sel[i] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const unsigned long long m = __ballot(s[u] == e);
+      if (s[u] == e) list[(size_t)e * T + c + __popcll(m & below)] = i0 + 64 * u + lane;
+      c += __popcll(m);
+    }
+  }
+  if (lane == 0) cnt[e] = c;
 }
 
 // The router in one workgroup for a decode batch (T <= 16 tokens, E <= 16 experts, D <= 4096):
@@ -614,6 +643,24 @@ static long long fmt_scale_halves(int fmt, long long rows, int K) {
        : fmt == FMT_Q4K ? rows * (K / 256) * 10 : fmt == FMT_Q6K ? rows * (K / 32) * 6 : rows;
 }
 
+// Expert linears on the split GEMM (afx_gemm_split.h): batches of more than 16 tokens, whose weights the
+// skinny kernels would stream once per 16 tokens of an expert, and from 4 tokens the formats without a
+// skinny MFMA kernel.  Pointers it cannot take stay on the other kernels.
+static bool moe_split_ok(int fmt, int T, int N, int K, const void* w, const void* scale, const void* x) {
+  const uintptr_t align = fmt == FMT_L4 ? 15 : fmt == FMT_I8 ? 1 : 3;
+  return T > (mfma_supported(fmt, K) ? 16 : 3) && split_supported(fmt, N, K) && w && x && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 &&
+         (fmt == FMT_F16 || (scale && ((uintptr_t)scale & align) == 0));
+}
+static int moe_split(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int N, int K,
+                     const int* cnt, const int* list, void* y, int ldy, int epi, hipStream_t stream, const char* what) {
+  SplitArgs a = {};
+  a.w = w; a.scale = (const half_t*)scale; a.x = (const half_t*)x; a.y = y;
+  a.w_es = fmt_row_bytes(fmt, K) * N; a.s_es = fmt_scale_halves(fmt, N, K);
+  a.cnt = cnt; a.list = list; a.T = T; a.E = E; a.topk = k; a.x_by_token = epi == EPI_SWIGLU;
+  a.ldx = K; a.ldy = ldy; a.N = N; a.K = K; a.epi = epi;
+  return split_moe_launch(fmt, a, stream, what);
+}
+
 }  // namespace afx
 
 using namespace afx;
@@ -686,15 +733,23 @@ int afx_moe_topk(const float* logits, int T, int E, int k, int renorm, float* ga
   const int jn = (E + 63) / 64;
   auto fn = jn <= 1 ? moe_topk_kernel<1> : jn <= 2 ? moe_topk_kernel<2> : jn <= 4 ? moe_topk_kernel<4>
           : jn <= 8 ? moe_topk_kernel<8> : jn <= 16 ? moe_topk_kernel<16> : moe_topk_kernel<33>;
-  const int waves = T < 16 ? T : 16;               // one wavefront per token, up to 16 at a time
-  hipLaunchKernelGGL(fn, dim3(1), dim3(64 * waves), (size_t)T * k * sizeof(int), (hipStream_t)stream,
-                     logits, T, E, k, renorm, gate, sel, cnt, list);
-  return check_launch("afx_moe_topk");
+  // one wavefront per token; up to 32 tokens one workgroup also makes the lists, more take four tokens
+  // per workgroup and a launch of their own for the lists
+  const int many = T > 32;
+  const int waves = many ? 4 : T < 16 ? T : 16;
+  hipLaunchKernelGGL(fn, dim3(many ? (T + 3) / 4 : 1), dim3(64 * waves), many ? 0 : (size_t)T * k * sizeof(int),
+                     (hipStream_t)stream, logits, T, E, k, renorm, many, gate, sel, cnt, list);
+  const int rc = check_launch("afx_moe_topk");
+  if (rc || !many) return rc;
+  hipLaunchKernelGGL(moe_bucket_kernel, dim3((E + 3) / 4), dim3(256), 0, (hipStream_t)stream, sel, T, E, k, cnt, list);
+  return check_launch("afx_moe_topk(lists)");
 }
 
 // W: [E][2F][D] gate/up interleaved rows (format fmt), x: normed hidden [T][D].
 int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int F, int D,
                    const int* cnt, const int* list, void* act, int rows_hint, void* stream) {
+  if (rows_hint == 0 && moe_split_ok(fmt, T, 2 * F, D, w, scale, x))
+    return moe_split(fmt, w, scale, x, T, k, E, 2 * F, D, cnt, list, act, F, EPI_SWIGLU, (hipStream_t)stream, "afx_moe_gateup");
   if (rows_hint == 0 && mfma_supported(fmt, D) && F % 2 == 0) {
     MfmaArgs m = {};
     m.w = w; m.scale = (const half_t*)scale; m.x = (const half_t*)x; m.ldx = D; m.y = act; m.ldy = F;
@@ -717,6 +772,8 @@ int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int
 int afx_moe_down(int fmt, const void* w, const void* scale, const void* act, int T, int k, int E, int F, int D,
                  const int* cnt, const int* list, float* y, int rows_hint, void* ws, long long ws_bytes,
                  void* stream) {
+  if (rows_hint == 0 && moe_split_ok(fmt, T, D, F, w, scale, act))
+    return moe_split(fmt, w, scale, act, T, k, E, D, F, cnt, list, y, D, EPI_F32, (hipStream_t)stream, "afx_moe_down");
   if (rows_hint == 0 && mfma_supported(fmt, F) && D % 4 == 0) {
     MfmaArgs m = {};
     m.w = w; m.scale = (const half_t*)scale; m.x = (const half_t*)act; m.ldx = F; m.y = y; m.ldy = D;
@@ -779,7 +836,7 @@ int afx_moe_down_combine(int fmt, const void* w, const void* scale, const void* 
                          const void* h, const float* gate, const void* shared, void* out, void* stream) {
   AFX_REQUIRE(h && gate && out && y, "afx_moe_down_combine: null pointer");
   int S = 1;
-  if (mfma_supported(fmt, F) && D % 4 == 0) {
+  if (mfma_supported(fmt, F) && D % 4 == 0 && !moe_split_ok(fmt, T, D, F, w, scale, act)) {
     MfmaArgs m = {};
     m.w = w; m.scale = (const half_t*)scale; m.x = (const half_t*)act; m.ldx = F; m.y = y; m.ldy = D;
     m.cnt = cnt; m.list = list; m.T = T; m.k = k; m.x_by_token = 0; m.N = D; m.K = F; m.epi = EPI_F32;

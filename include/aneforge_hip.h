@@ -263,6 +263,18 @@ int afx_moe_down_combine(int fmt, const void* w, const void* scale, const void* 
  * residual, 2 fp32, 3 SwiGLU over interleaved gate/up rows (aneforge/llm.py:171-175). */
 int afx_gemm(int fmt, const void* w, const void* scale, const void* x, int ldx, void* y, int ldy, int M, int N,
              int K, const void* bias, const void* residual, int epi, void* stream);
+/* The same linear over any packed weight format (fmt 0..6), decoded in the kernel: N % 16 == 0, K % 128 == 0
+ * (256 for Q4_K / Q6_K).  ws (optional, 16-byte aligned, may be NULL): an fp32 workspace; with the bytes
+ * afx_gemm_split_plan asks for, the reduction is cut into K slices whose partials meet there and a second
+ * launch sums them, with fewer bytes the slices are fewer.  Results differ from afx_gemm only in fp32
+ * summation order.  The reference has one matmul for any row count (aneforge/_compile.py:375-385). */
+int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int ldx, void* y, int ldy, int M, int N,
+                   int K, const void* bias, const void* residual, int epi, void* ws, long long ws_bytes,
+                   void* stream);
+/* 1 where afx_gemm_split is the faster of the two (for formats afx_gemm does not read: than afx_dequant_f16 +
+ * afx_gemm), which is up to a few hundred rows, or more for the 4-bit formats; 0 where it is not; negative for
+ * shapes it does not take.  *ws_bytes (optional): the workspace of its slices. */
+int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes);
 /* prompt [q | k | v] rows -> RoPE'd q and K/V cache rows at pos0.. (aneforge/llm.py:96-105, 149-168) */
 int afx_qkv_split_rope(const void* qkv, int ldqkv, int M, int nq, int nk, int dh, const void* cos_tab,
                        const void* sin_tab, int pos0, int rope, void* q, int ldq, void* kcache, void* vcache,

@@ -1,0 +1,211 @@
+"""The split GEMM (every packed format, row tiles, K slices and K groups) and the grouped experts on it,
+against fp64 products with the oracle's dequantised weights.
+
+Bar: an output differs from the fp64 product by its own rounding (half an fp16 ulp, 2^-11 relative) and
+by the fp32 accumulation, at most K * 2^-24 of the sum of the terms' magnitudes; the SwiGLU epilogue
+rounds gate and up to fp16 first and takes the repository's fp16 bar."""
+import os
+
+import numpy as np
+import pytest
+
+from _util import check_f16, check_hidden, dev, host, say
+from oracle import ref
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+FMTS = ["int8", "q4_0", "fp16", "blockwise", "lut4", "q4_k", "q6_k"]
+
+
+@pytest.fixture(scope="module")
+def K():
+    from aneforge_amd import _kernels
+    return _kernels
+
+
+def _weights(K, fmt, N, Kd, rng):
+    """(codes, scale, fp64 weights) of a random [N, Kd] matrix on the device."""
+    if fmt == "int8":
+        q = rng.integers(-127, 128, (N, Kd), dtype=np.int8)
+        s = (np.abs(rng.normal(0, 0.02, N)) / 127 + 1e-5).astype(np.float16)
+        return dev(q), dev(s), ref.dequant_w8(q, s).astype(np.float64)
+    if fmt == "fp16":
+        w = (rng.standard_normal((N, Kd)) * 0.02).astype(np.float16)
+        return dev(w), None, w.astype(np.float64)
+    if fmt == "blockwise":
+        q = rng.integers(-127, 128, (N, Kd), dtype=np.int8)
+        s = (np.abs(rng.normal(0, 0.02, (N, Kd // 32))) / 127 + 1e-5).astype(np.float16)
+        return dev(q), dev(s), ref.dequant_blockwise(q, s).astype(np.float64)
+    if fmt == "lut4":
+        packed = rng.integers(0, 256, (N, Kd // 2), dtype=np.uint8)
+        cb = np.sort(rng.normal(0, 0.02, (N, 16)), axis=1).astype(np.float16)
+        idx = np.empty((N, Kd), np.int64)
+        idx[:, 0::2], idx[:, 1::2] = packed & 15, packed >> 4
+        return dev(packed), dev(cb), np.take_along_axis(cb.astype(np.float64), idx, axis=1)
+    if fmt == "q4_0":
+        b = ref.quantize_q4_0((rng.standard_normal((N, Kd)) * 0.05).astype(np.float32))
+        return (*K.q4_repack(dev(b), N, Kd), ref.dequant_q4_0_f16(b, N, Kd).astype(np.float64))
+    nb = N * Kd // 256
+    if fmt == "q4_k":
+        b = rng.integers(0, 256, (nb, 144), dtype=np.uint8)
+        b[:, :4] = (np.abs(rng.standard_normal((nb, 2))) * 0.0005 + 1e-5).astype(np.float16).view(np.uint8).reshape(nb, 4)
+        b = b.reshape(N, -1)
+        return (*K.q4_k_repack(dev(b), N, Kd), ref.dequant_q4_k_f16(b, N, Kd).astype(np.float16).astype(np.float64))
+    b = rng.integers(0, 256, (nb, 210), dtype=np.uint8)
+    b[:, 208:210] = (np.abs(rng.standard_normal(nb)) * 0.0005 + 1e-5).astype(np.float16).view(np.uint8).reshape(nb, 2)
+    b = b.reshape(N, -1)
+    return (*K.q6_k_repack(dev(b), N, Kd), ref.dequant_q6_k_f16(b, N, Kd).astype(np.float16).astype(np.float64))
+
+
+def _bound(x, W, want):
+    mag = np.abs(x.astype(np.float64)) @ np.abs(W).T
+    return np.abs(want) * 2.0 ** -11 + mag * W.shape[1] * 2.0 ** -24 + 2.0 ** -24
+
+
+# (slices, features / 32, row tiles / 16): every kernel built, the slice counts around the K = 1280 row's ten
+# chunks (one short slice, one chunk each), and more than one row tile
+CONFIGS = [(1, 2, 1), (3, 4, 1), (10, 2, 2), (2, 4, 2), (4, 2, 3), (1, 4, 3), (16, 2, 4), (1, 4, 4), (3, 2, 6), (2, 4, 6),
+           (1, 2, 8), (7, 4, 8)]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_every_tile_and_slice_count(K, fmt, monkeypatch):
+    rng = np.random.default_rng(len(fmt))
+    N, Kd = 16 * 17, 1280                                   # a ragged feature tile, K not a power of two
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    ws = torch.empty(16 * 256 * 512, dtype=torch.float32, device="cuda")
+    cfgs = CONFIGS + ([(1, 8, 4), (2, 8, 6)] if fmt in ("int8", "q4_0") else []) + ([(1, 8, 8), (5, 8, 8)] if fmt == "int8" else [])
+    for S, nw, mt in cfgs:
+        M = 16 * mt + 5 if S % 2 else 16 * mt - 3           # past one row tile, and short of it
+        x = rng.standard_normal((M, Kd)).astype(np.float16)
+        want = x.astype(np.float64) @ W.T
+        say(f"gemm_split {fmt} M={M} N={N} K={Kd} slices={S} nw={nw} mt={mt}")
+        monkeypatch.setenv("AFX_GEMM_SPLIT", f"{S}.{nw}.{mt}")
+        y = torch.full((M, N), 7.0, dtype=torch.float16, device="cuda")
+        K.gemm_split(fmt, w, s, dev(x), y, ws=ws)
+        got = host(y)
+        assert (np.abs(got - want) <= _bound(x, W, want)).all(), (S, nw, mt)
+        again = torch.empty_like(y)
+        K.gemm_split(fmt, w, s, dev(x), again, ws=ws)       # the slices' sum has a fixed order
+        assert np.array_equal(host(again).view(np.uint16), got.view(np.uint16))
+
+
+@pytest.mark.parametrize("fmt", ["int8", "q4_k"])
+@pytest.mark.parametrize("cfg", ["1.2.2", "5.4.2"])
+@pytest.mark.parametrize("ldy_pad", [0, 5])                 # 5: rows that take no 8- or 16-byte stores
+def test_epilogues(K, fmt, cfg, ldy_pad, monkeypatch):
+    monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
+    rng = np.random.default_rng(7 + ldy_pad)
+    M, N, Kd = 37, 96, 768
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    xp = torch.zeros((M, Kd + 16), dtype=torch.float16, device="cuda")
+    xp[:, :Kd] = dev(x)
+    bias = (rng.standard_normal(N) * 0.1).astype(np.float16)
+    r = rng.standard_normal((M, N)).astype(np.float16)
+    ws = torch.empty(8 * 128 * 64, dtype=torch.float32, device="cuda")
+    lin = x.astype(np.float64) @ W.T
+    say(f"gemm_split epilogues {fmt} cfg={cfg} ldy+{ldy_pad}")
+
+    def out(cols, dtype=torch.float16):
+        return torch.zeros((M, cols + ldy_pad), dtype=dtype, device="cuda")[:, :cols]
+    y = K.gemm_split(fmt, w, s, xp[:, :Kd], out(N), bias=dev(bias), ws=ws)
+    want = lin + bias.astype(np.float64)
+    assert (np.abs(host(y) - want) <= _bound(x, W, want) + np.abs(lin) * 2.0 ** -23).all()
+    y = K.gemm_split(fmt, w, s, xp[:, :Kd], out(N, torch.float32), epi="f32", ws=ws)
+    assert (np.abs(host(y) - lin) <= _bound(x, W, lin)).all()
+    y = out(N)
+    y.copy_(dev(r))
+    K.gemm_split(fmt, w, s, xp[:, :Kd], y, residual=y, epi="resid", ws=ws)
+    check_hidden(host(y), ref.r16(r.astype(np.float64) + ref.r16(lin)), what="resid")
+    y = K.gemm_split(fmt, w, s, xp[:, :Kd], out(N // 2), epi="swiglu", ws=ws)
+    check_f16(host(y), ref.r16(ref.silu(ref.r16(lin[:, 0::2])) * ref.r16(lin[:, 1::2])), what="swiglu")
+
+
+def test_workspace_limits_the_slices_and_bad_shapes_raise(K, monkeypatch):
+    rng = np.random.default_rng(3)
+    w, s, W = _weights(K, "int8", 64, 512, rng)
+    x = rng.standard_normal((20, 512)).astype(np.float16)
+    want = x.astype(np.float64) @ W.T
+    monkeypatch.setenv("AFX_GEMM_SPLIT", "4.2.2")
+    per = 2 * 2 * 2048                                      # bytes of one slice: mt * nw * 2 KB tiles
+    for nbytes in (0, 2 * per, 3 * per + 8, 4 * per):
+        ws = torch.empty(nbytes // 4, dtype=torch.float32, device="cuda") if nbytes else None
+        guard = torch.full((20, 64), 7.0, dtype=torch.float16, device="cuda")
+        y = K.gemm_split("int8", w, s, dev(x), guard, ws=ws)
+        assert (np.abs(host(y) - want) <= _bound(x, W, want)).all(), nbytes
+    with pytest.raises(RuntimeError, match="K %"):
+        K.gemm_split("int8", w[:, :64].contiguous(), s, dev(x[:, :64].copy()), torch.empty((20, 64), dtype=torch.float16, device="cuda"))
+    monkeypatch.delenv("AFX_GEMM_SPLIT")
+    assert K.gemm_split_plan("int8", 20, 64, 64) == (False, 0)      # K = 64: afx_gemm's
+    assert K.gemm_split_plan("q4_0", 64, 4096, 4096)[0]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("E,T,k", [(3, 70, 2), (130, 33, 2), (5, 4, 3)])
+def test_grouped_experts(K, fmt, E, T, k):
+    """Skewed routing: one expert takes every token (several row tiles), others one row, some none; 130
+    experts need more than one pass over the counts; 4 tokens where the format has no skinny MFMA kernel."""
+    rng = np.random.default_rng(E + T)
+    D, F = 512, 256
+    say(f"grouped experts {fmt} E={E} T={T} k={k}")
+    used = [E - 1] + [int(e) for e in rng.choice(E - 1, min(E - 1, 4), replace=False)]
+    pick = [[E - 1] + [int(e) for e in rng.choice(used[1:], k - 1, replace=False)] for _ in range(T)]
+    cnt, lst = np.zeros(E, np.int32), np.zeros((E, T), np.int32)
+    for t in range(T):
+        for sl, e in enumerate(pick[t]):
+            lst[e, cnt[e]] = t * k + sl
+            cnt[e] += 1
+    gu, gus, G = [], [], {}
+    dn, dns, Dn = [], [], {}
+    zero_g, zero_d = _weights(K, fmt, 2 * F, D, rng), _weights(K, fmt, D, F, rng)
+    for e in range(E):
+        a, b = (_weights(K, fmt, 2 * F, D, rng), _weights(K, fmt, D, F, rng)) if e in used else (zero_g, zero_d)
+        gu.append(a[0]); gus.append(a[1]); G[e] = a[2]
+        dn.append(b[0]); dns.append(b[1]); Dn[e] = b[2]
+    cat = lambda ts: None if ts[0] is None else torch.cat(ts)
+    x = (rng.standard_normal((T, D)) * 0.5).astype(np.float16)
+    act = K.moe_gateup(fmt, cat(gu), cat(gus), dev(x), k, E, F, dev(cnt), dev(lst))
+    a = host(act)
+    y = host(K.moe_down(fmt, cat(dn), cat(dns), act, T, k, E, F, D, dev(cnt), dev(lst)))
+    for t in range(T):
+        for sl, e in enumerate(pick[t]):
+            lin = ref.r16(x[t].astype(np.float64) @ G[e].T)
+            i = t * k + sl
+            check_f16(a[i], ref.r16(ref.silu(lin[0::2]) * lin[1::2]), what=f"gate/up token {t} expert {e}")
+            want = a[i].astype(np.float64) @ Dn[e].T
+            assert (np.abs(y[i] - want) <= _bound(a[i][None], Dn[e], want[None])[0]).all(), (t, e)
+
+
+@pytest.mark.parametrize("T,E,k", [(33, 8, 2), (300, 8, 2), (65, 130, 4), (64, 3, 3)])
+def test_topk_lists_of_many_tokens(K, T, E, k):
+    """More than 32 tokens: the gates, choices and lists are those of the one-workgroup form on 32 tokens
+    at a time, joined in token order."""
+    say(f"moe_topk T={T} E={E} k={k}")
+    rng = np.random.default_rng(T)
+    lg = np.round(rng.standard_normal((T, E)).astype(np.float32), 1)     # ties
+    gate, sel, cnt, lst = (host(t) for t in K.moe_topk(dev(lg), k, True))
+    gates, sels, joined = [], [], [[] for _ in range(E)]
+    for t0 in range(0, T, 32):
+        g, s, c, l = (host(t) for t in K.moe_topk(dev(lg[t0:t0 + 32]), k, True))
+        gates.append(g); sels.append(s)
+        for e in range(E):
+            joined[e] += [int(i) + t0 * k for i in l[e, :c[e]]]
+    assert np.array_equal(gate.view(np.uint32), np.concatenate(gates).view(np.uint32))
+    assert np.array_equal(sel, np.concatenate(sels))
+    for e in range(E):
+        assert cnt[e] == len(joined[e]) and lst[e, :cnt[e]].tolist() == joined[e]
+
+
+@pytest.mark.parametrize("M", [17, 300])
+def test_router_rows_past_16(K, M):
+    """A linear with few outputs and many rows: the row groups run in workgroups of their own."""
+    say(f"fp16 router rows M={M}")
+    rng = np.random.default_rng(M)
+    w, _, W = _weights(K, "fp16", 8, 4096, rng)
+    x = rng.standard_normal((M, 4096)).astype(np.float16)
+    want = x.astype(np.float64) @ W.T
+    got = host(K.linear("fp16", w, None, dev(x), out_f32=True))
+    assert (np.abs(got - want) <= _bound(x, W, want)).all()
