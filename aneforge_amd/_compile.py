@@ -479,12 +479,32 @@ class _Lowering:
                                                M * Kd if ba > 1 else 0, Kd * N if bb > 1 else 0, M * N,
                                                K.stream()))
 
+    @staticmethod
+    def _sdpa_on_mfma(H, Sq, Skv, D):
+        """Whether unmasked attention runs on the MFMA kernel (afx_sdpa) rather than the decode kernel, by
+        their predicted microseconds.  The decode kernel streams every key for every query (8 M
+        multiply-adds a microsecond: 32 heads x 512 x 512 x 128 measured 129); the MFMA kernel walks
+        64-key blocks, two halves at once, per 64 queries of a head, one workgroup a CU (2.85 us a block at
+        D = 128, 2.0 at 64: the same shape 17).  Few queries over many keys stay on the split-KV kernel."""
+        if D not in (64, 128):
+            return False
+        blocks = -(-(-(-Skv // 64)) // 2)
+        rounds = -(-(H * -(-Sq // 64)) // 256)
+        base, block = (4.0, 2.85) if D == 128 else (3.4, 2.0)
+        return base + block * blocks * rounds < 5.0 + H * Sq * Skv * D / 8e6
+
     def _op_sdpa(self, t):
         q, k, v = (self.buf[id(s)] for s in t.srcs[:3])
         mask = self.buf[id(t.srcs[3])] if t.attrs.get("masked") else None
         _, H, Sq, D = t.srcs[0].shape
         _, Hkv, Skv, _ = t.srcs[1].shape
         y = self.out(t)
+        if (mask is None and self._sdpa_on_mfma(H, Sq, Skv, D)
+                and all(b.is_contiguous() and b.data_ptr() % 16 == 0 for b in (q, k, v, y))):
+            qh, kh, vh, yh = q.view(H, Sq, D), k.view(Hkv, Skv, D), v.view(Hkv, Skv, D), y.view(H, Sq, D)
+            scale, causal = t.attrs["scale"], bool(t.attrs.get("causal"))
+            self.steps.append(lambda: K.sdpa(qh, kh, vh, yh, scale, causal))
+            return
         causal_off = (Skv - Sq) if t.attrs.get("causal") else -1
         ws = torch.zeros(K.attn_ws_bytes(Sq, H, Hkv, D, Skv) // 4 + 1, dtype=torch.float32, device="cuda")
         self.keep.append(ws)

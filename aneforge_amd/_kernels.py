@@ -194,6 +194,17 @@ def decode_attn(q, k, v, o=None, ctx_len=None, pos=None, scale=None, mask=None, 
     return o
 
 
+def sdpa(q, k, v, o, scale, causal=False):
+    """o = softmax(q k^T * scale) v for contiguous q/o [.., H, Sq, D] and k/v [.., Hkv, Skv, D] (see afx_sdpa)."""
+    _dev(q, k, v, o)
+    H, Sq, D = q.shape[-3:]
+    Hkv, Skv = k.shape[-3:-1]
+    if k.shape != v.shape or k.shape[-1] != D or o.shape != q.shape or not all(t.is_contiguous() for t in (q, k, v, o)):
+        raise ValueError("sdpa: q/o [H, Sq, D] and k/v [Hkv, Skv, D] must match and be contiguous")
+    _hip.call("afx_sdpa", P(q), P(k), P(v), P(o), H, Hkv, Sq, Skv, D, int(bool(causal)), float(scale), stream())
+    return o
+
+
 # --------------------------------------------------------------------------- small ops
 def rmsnorm(x, gamma, eps, y=None):
     _dev(x, gamma)

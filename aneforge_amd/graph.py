@@ -253,8 +253,8 @@ def sdpa(q: Tensor, k: Tensor, v: Tensor, scale: float | None = None, is_causal:
          attn_mask: Tensor | None = None) -> Tensor:
     """softmax(q k^T * scale (+ mask)) v for q [1, H, Sq, D], k/v [1, Hkv, Skv, D]
     (aneforge/graph.py:993-1040).  Validation follows the reference; grouped-query k/v
-    (H a multiple of Hkv) is accepted in addition.  The device kernel is split-KV decode
-    attention for every regime, so there is no native/decomposed switch."""
+    (H a multiple of Hkv) is accepted in addition.  There is no native/decomposed switch: the
+    compiler takes the split-KV decode kernel or, for many unmasked queries, the MFMA one."""
     if not (len(q.shape) == 4 == len(k.shape) == len(v.shape)):
         raise ValueError(f"af.sdpa expects 4D q,k,v of [1,H,S,D]; got {q.shape}, {k.shape}, {v.shape}")
     if k.shape != v.shape:

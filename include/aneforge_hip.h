@@ -153,6 +153,12 @@ int afx_decode_attn_noalloc(const void* q, const void* k, const void* v, void* o
                             int ctx_len, const int* pos, int max_len, const void* mask, long long mask_bs,
                             int causal_off, float scale, int nstep_hint, void* stream);
 
+/* af.sdpa over many queries (aneforge/graph.py:993-1040): o = softmax(q k^T * scale) v for contiguous fp16
+ * q / o [H][Sq][D], k / v [Hkv][Skv][D], D 64 or 128, query head h on kv head h / (H / Hkv); causal: query i
+ * sees keys 0 .. Skv - Sq + i (Skv >= Sq).  On MFMA with the probabilities kept to 22 bits. */
+int afx_sdpa(const void* q, const void* k, const void* v, void* o, int H, int Hkv, int Sq, int Skv, int D, int causal,
+             float scale, void* stream);
+
 /* ---- norms, rope, sampling -------------------------------------------------------------- */
 
 /* (aneforge/graph.py:293-301) */

@@ -250,3 +250,12 @@ def test_reference_import_name_resolves_to_this_build():
     assert aneforge.compile is aneforge_amd.compile and aneforge.LlamaPrefill is aneforge_amd.LlamaPrefill
     assert LP is aneforge_amd.llm.LlamaPrefill and load_gguf is aneforge_amd.moe.load_gguf
     assert g.GGUFView is aneforge_amd.GGUFView and aneforge.sdpa is aneforge_amd.sdpa
+
+
+def test_sdpa_kernel_choice():
+    """Many queries go to the MFMA attention, few queries (over any number of keys) and other head dims
+    to the decode kernel."""
+    from aneforge_amd._compile import _Lowering
+    on = _Lowering._sdpa_on_mfma
+    assert on(32, 512, 512, 128) and on(4, 1500, 1500, 64) and on(8, 128, 128, 128) and on(32, 64, 64, 64)
+    assert not on(8, 1, 8192, 128) and not on(4, 16, 8192, 128) and not on(32, 4, 300, 64) and not on(32, 512, 512, 96)
