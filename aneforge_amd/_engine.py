@@ -242,6 +242,12 @@ def gemm_plan(fmt: str, M: int, N: int, Kd: int):
     return K.gemm_split_plan(fmt, M, N, Kd)
 
 
+@functools.lru_cache(maxsize=4096)
+def attn_plan(M: int, pos0: int, H: int, KV: int, dh: int):
+    """(key ranges, workspace bytes) of the prompt rows' attention: see K.prefill_attn_plan."""
+    return K.prefill_attn_plan(M, pos0, H, KV, dh)
+
+
 def prefill_gemm(eng, lin: "Linear", x, y, residual=None, epi="f16"):
     """The batched prefill's linear.  The split GEMM reads every packed format and cuts K over the
     chip; it is taken where its plan is the faster (up to a few hundred rows, further for the 4-bit
@@ -374,7 +380,11 @@ class AttentionDecode:
             K.head_norm_rope(self.kc[0], KV, dh, self.k_norm, self.eps, eng.cos, eng.sin, pos, seq_stride=0,
                              head_stride=self.kc.stride(1), pos_mul=dh, kv_len=eng.M, M=m, rope=self.rope)
         a = bufs["a"][:m, :H * dh]
-        K.prefill_attn(q, self.kc[0], self.vc[0], a, pos0, H, KV)
+        ranges, ws_bytes = attn_plan(m, pos0, H, KV, dh)
+        if ranges > 1:
+            K.prefill_attn_split(q, self.kc[0], self.vc[0], a, pos0, H, KV, ranges, eng.gemm_scratch(ws_bytes))
+        else:
+            K.prefill_attn(q, self.kc[0], self.vc[0], a, pos0, H, KV)
         prefill_gemm(eng, self.wo, a, X, residual=X, epi="resid")
 
     @property
@@ -620,8 +630,8 @@ class DecodeEngine:
         return self._w16[:n]
 
     def gemm_scratch(self, nbytes: int) -> torch.Tensor:
-        """An fp32 workspace of at least nbytes for the split GEMM's partials (reused by every linear in
-        stream order; a prompt's largest is a few MB per hundred rows)."""
+        """An fp32 workspace of at least nbytes for the split GEMM's and the split attention's partials
+        (reused by every launch in stream order; a prompt's largest is a few MB per hundred rows)."""
         if getattr(self, "_gws", None) is None or self._gws.numel() * 4 < nbytes:
             self._gws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device="cuda")
         return self._gws

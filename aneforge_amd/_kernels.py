@@ -516,3 +516,20 @@ def prefill_attn(q, kcache, vcache, o, pos0, Hq, Hkv, scale=None):
     _hip.call("afx_prefill_attn", P(q), q.stride(0), P(kcache), P(vcache), kcache.stride(-3), kcache.shape[-2],
               P(o), o.stride(0), M, int(pos0), Hq, Hkv, D, scale, stream())
     return o
+
+
+def prefill_attn_plan(M, pos0, Hq, Hkv, D):
+    """(key ranges prefill_attn_split should cut, 1 where prefill_attn is the faster; workspace bytes)."""
+    n = C.c_longlong(0)
+    return _hip.call("afx_prefill_attn_plan", M, int(pos0), Hq, Hkv, D, C.byref(n)), n.value
+
+
+def prefill_attn_split(q, kcache, vcache, o, pos0, Hq, Hkv, ranges, ws, scale=None):
+    """prefill_attn with each query tile's keys cut into `ranges` parts (see afx_prefill_attn_split); ws: fp32."""
+    _dev(q, kcache, vcache, o, ws)
+    M = q.shape[0]
+    D = kcache.shape[-1]
+    scale = 1.0 / float(np.sqrt(D)) if scale is None else float(scale)
+    _hip.call("afx_prefill_attn_split", P(q), q.stride(0), P(kcache), P(vcache), kcache.stride(-3), kcache.shape[-2],
+              P(o), o.stride(0), M, int(pos0), Hq, Hkv, D, scale, int(ranges), P(ws), _nbytes(ws), stream())
+    return o

@@ -16,6 +16,7 @@
 // consecutive keys of one dim).  S stays in registers for an online softmax (row max and sum
 // by DPP rotations inside the 16-lane rows that hold one query row's scores); P goes through a
 // wavefront-private LDS tile to change from the MFMA result layout to the operand layout.
+#include <math.h>
 #include <stdlib.h>
 #include "afx_common.h"
 
@@ -885,6 +886,125 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// ---- form 3 with the keys cut over several workgroups ----
+// A few query rows over a long cache (verification rows, a chat turn, a prompt's last chunk) are one or
+// two tiles per head: 32 workgroups walk the whole cache at 1.5 us per 64-key block (2048 rows: 57 us at
+// any M up to 100).  Here a workgroup takes one of S ranges of a tile's key blocks and leaves fp32
+// accumulators, running maxima and sums; the second launch weighs and adds them.  100 rows at position
+// 2048: 62.6 -> 28 us, 8 rows 55.7 -> 19.  Arithmetic of a block as form 3.
+struct AttnSplitArgs {
+  float* po;               // [S][Hq][M][128]
+  float* ml;               // [S][Hq][M][2]
+  int S;
+};
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attn_split_kernel(PrefillAttnArgs a,
+                                                                                                            AttnSplitArgs sa) {
+  __shared__ __align__(16) unsigned char Ks[2][kPK * kKStride];
+  __shared__ __align__(16) unsigned char Vt[2][kPK * kVRow];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int fr = lane & 15, fg = lane >> 4;
+  const int id = blockIdx.x, G = a.Hq / a.Hkv;
+  int t, h, sl;                                  // tile, head and key range; kv head k on XCD k % 8
+  if (a.xcd_map) {
+    const int x = id & 7, l = id >> 3, per_t = (a.Hkv >> 3) * G;
+    sl = l % sa.S;
+    const int r = l / sa.S % per_t;
+    t = l / sa.S / per_t;
+    h = (x + 8 * (r / G)) * G + r % G;
+  } else {
+    sl = id % sa.S;
+    h = id / sa.S % a.Hq;
+    t = id / sa.S / a.Hq;
+  }
+  const int m0 = t * kPQ3, kvh = h / G;
+  const int mlast = m0 + kPQ3 - 1 < a.M - 1 ? m0 + kPQ3 - 1 : a.M - 1;
+  const int nkb = (a.pos0 + mlast) / kPK + 1;
+  const int kb0 = nkb * sl / sa.S, kb1 = nkb * (sl + 1) / sa.S;
+  const int mw = m0 + 32 * wave;
+  const int wlast = mw < a.M ? a.pos0 + (mw + 31 < a.M - 1 ? mw + 31 : a.M - 1) : -1;
+  const half_t* kbase = a.k + (size_t)kvh * a.kv_hs;
+  const half_t* vbase = a.v + (size_t)kvh * a.kv_hs;
+  KvRegs r;
+  if (kb0 < kb1) kv_load_rm(a, kbase, vbase, kb0 * kPK, tid, r);
+  h8 qf[2][4];
+  int qp[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int mq = mw + 16 * u + fr;
+    const half_t* qrow = a.q + (size_t)(mq < a.M ? mq : a.M - 1) * a.ldq + (size_t)h * kPD;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[u][ks] = __builtin_bit_cast(h8, *(const u4*)(qrow + ks * 32 + 8 * fg));
+    qp[u] = a.pos0 + mq;
+  }
+  f4 acc[2][8];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[u][d] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+  float mrow[2] = {-INFINITY, -INFINITY}, lrow[2] = {0.0f, 0.0f};
+  if (kb0 < kb1) kv_stage_rm(r, Ks[0], Vt[0], tid);
+  __syncthreads();
+  for (int kb = kb0; kb < kb1; ++kb) {
+    const int s = (kb - kb0) & 1;
+    if (kb + 1 < kb1) kv_load_rm(a, kbase, vbase, (kb + 1) * kPK, tid, r);
+    if (kb * kPK <= wlast)                       // blocks wholly past the wavefront's queries are skipped
+      attn_block3<true, true>(a, Ks[s], Vt[s], qf, qp, kb * kPK, a.pos0 + mw, fr, fg, acc, mrow, lrow);
+    if (kb + 1 < kb1) kv_stage_rm(r, Ks[s ^ 1], Vt[s ^ 1], tid);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int m = mw + 16 * u + fr;
+    if (m >= a.M) continue;
+    const size_t row = ((size_t)sl * a.Hq + h) * a.M + m;
+    if (fg == 0) *(float2*)(sa.ml + 2 * row) = float2{mrow[u], lrow[u]};
+    if (kb0 < kb1) {                             // an empty range's weight is 0: its accumulators are not read
+#pragma unroll
+      for (int d = 0; d < 8; ++d) *(f4*)(sa.po + row * kPD + d * 16 + 4 * fg) = acc[u][d];
+    }
+  }
+}
+__global__ __launch_bounds__(256) void prefill_attn_merge_kernel(PrefillAttnArgs a, AttnSplitArgs sa) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // 32 threads of 4 dims per row
+  const long long rows = (long long)a.Hq * a.M;
+  if (i >= rows * 32) return;
+  const long long row = i >> 5;
+  const int d = (int)(i & 31) * 4;
+  float mx = -INFINITY;
+  for (int s = 0; s < sa.S; ++s) mx = fmaxf(mx, sa.ml[2 * (s * rows + row)]);
+  float l = 0.0f;
+  f4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < sa.S; ++s) {
+    const float2 p = *(const float2*)(sa.ml + 2 * (s * rows + row));
+    if (p.x == -INFINITY) continue;              // no key of the range seen
+    const float w = __builtin_amdgcn_exp2f(p.x - mx);
+    l += w * p.y;
+    const f4 v = *(const f4*)(sa.po + (s * rows + row) * kPD + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] += w * v[e];
+  }
+  const float inv = 1.0f / l;
+  half_t* op = a.o + (size_t)(row % a.M) * a.ldo + (size_t)(row / a.M) * kPD + d;
+  const h2 lo = {(half_t)(o[0] * inv), (half_t)(o[1] * inv)}, hi = {(half_t)(o[2] * inv), (half_t)(o[3] * inv)};
+  *(u2*)op = (u2){as_u32(lo), as_u32(hi)};
+}
+// Key ranges with the least predicted time (1: afx_prefill_attn's forms as they are): 1.5 us per 64-key
+// block and round of workgroups (two per CU), and for S > 1 the merge launch and 0.4 us per MB of partials.
+static int attn_split_ranges(int M, int pos0, int Hq) {
+  const double wgs = (double)((M + kPQ3 - 1) / kPQ3) * Hq;
+  const int nkb = (pos0 + M - 1) / kPK + 1;
+  // form 5 (pos0 < M) runs a tile's key halves side by side, one workgroup per CU
+  double best = pos0 < M ? 1.4 * ((nkb + 1) / 2) * ceil(wgs / 256) : 1.5 * nkb * ceil(wgs / 512);
+  best *= 0.9;
+  int S = 1;
+  for (int s = 2; s <= 16 && s <= nkb; ++s) {
+    const double us = 1.5 * ((nkb + s - 1) / s) * ceil(wgs * s / 512) + 3.5 + 0.4 * s * M * (double)Hq * kPD * 4e-6;
+    if (us < best) { best = us; S = s; }
+  }
+  return S;
+}
+static long long attn_split_bytes(int S, int M, int Hq) { return (long long)S * M * Hq * (kPD + 2) * 4; }
+
 }  // namespace afx
 
 using namespace afx;
@@ -963,6 +1083,49 @@ int afx_prefill_attn(const void* q, int ldq, const void* kcache, const void* vca
     }
   }
   return check_launch("afx_prefill_attn");
+}
+
+// Key ranges afx_prefill_attn_split cuts at this shape (1: it is not the faster form), with their workspace.
+int afx_prefill_attn_plan(int M, int pos0, int Hq, int Hkv, int D, long long* ws_bytes) {
+  if (ws_bytes) *ws_bytes = 0;
+  AFX_REQUIRE(D == kPD && M >= 1 && pos0 >= 0 && pos0 <= (1 << 30) && M <= (1 << 30) && Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0,
+              "afx_prefill_attn_plan: M=%d pos0=%d Hq=%d Hkv=%d D=%d not supported", M, pos0, Hq, Hkv, D);
+  const int S = attn_split_ranges(M, pos0, Hq);
+  if (ws_bytes && S > 1) *ws_bytes = attn_split_bytes(S, M, Hq);
+  return S;
+}
+
+int afx_prefill_attn_split(const void* q, int ldq, const void* kcache, const void* vcache, long long kv_hs, int Mmax,
+                           void* o, int ldo, int M, int pos0, int Hq, int Hkv, int D, float scale, int ranges, void* ws,
+                           long long ws_bytes, void* stream) {
+  AFX_REQUIRE(q && kcache && vcache && o && ws, "afx_prefill_attn_split: null pointer");
+  AFX_REQUIRE(D == kPD, "afx_prefill_attn_split: head dim %d not supported (128)", D);
+  AFX_REQUIRE(scale > 0.0f, "afx_prefill_attn_split: scale %g must be positive", (double)scale);
+  AFX_REQUIRE(Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0, "afx_prefill_attn_split: bad heads Hq=%d Hkv=%d", Hq, Hkv);
+  AFX_REQUIRE(M >= 1 && pos0 >= 0 && pos0 <= Mmax - M && kv_hs >= (long long)Mmax * D,
+              "afx_prefill_attn_split: %d positions from %d outside the %d-row cache", M, pos0, Mmax);
+  AFX_REQUIRE(ldq % 8 == 0 && ldq >= Hq * D && ldo % 4 == 0 && ldo >= Hq * D && kv_hs % 8 == 0 && ((uintptr_t)o & 7) == 0 &&
+              (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)ws) & 15) == 0,
+              "afx_prefill_attn_split: q / cache / workspace must be 16-byte aligned rows, o 8-byte");
+  AFX_REQUIRE(ranges >= 1 && ranges <= 64 && ws_bytes >= attn_split_bytes(ranges, M, Hq),
+              "afx_prefill_attn_split: %d key ranges need %lld workspace bytes", ranges, attn_split_bytes(ranges, M, Hq));
+  PrefillAttnArgs a = {};
+  a.q = (const half_t*)q; a.k = (const half_t*)kcache; a.v = (const half_t*)vcache; a.o = (half_t*)o;
+  a.kv_hs = kv_hs; a.ldq = ldq; a.ldo = ldo; a.M = M; a.pos0 = pos0; a.Hq = Hq; a.Hkv = Hkv; a.Mmax = Mmax;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  a.tiles = (M + kPQ3 - 1) / kPQ3;
+  a.xcd_map = Hkv % 8 == 0;
+  AttnSplitArgs sa = {};
+  sa.S = ranges;
+  sa.po = (float*)ws;
+  sa.ml = sa.po + (size_t)ranges * M * Hq * kPD;
+  const long long blocks = (long long)a.tiles * Hq * ranges, threads = (long long)M * Hq * 32;
+  AFX_REQUIRE(blocks < (1ll << 31) && threads < (1ll << 39), "afx_prefill_attn_split: too large");
+  hipLaunchKernelGGL(prefill_attn_split_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, sa);
+  const int rc = check_launch("afx_prefill_attn_split");
+  if (rc) return rc;
+  hipLaunchKernelGGL(prefill_attn_merge_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a, sa);
+  return check_launch("afx_prefill_attn_split(merge)");
 }
 
 }  // extern "C"

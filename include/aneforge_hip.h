@@ -289,6 +289,14 @@ int afx_qkv_split_rope(const void* qkv, int ldqkv, int M, int nq, int nk, int dh
  * GQA as _repeat_kv3, :205-211; softmax as aneforge/_bridges/ane_sdpa_fused.py:57-68) */
 int afx_prefill_attn(const void* q, int ldq, const void* kcache, const void* vcache, long long kv_hs, int Mmax,
                      void* o, int ldo, int M, int pos0, int Hq, int Hkv, int D, float scale, void* stream);
+/* The same attention with the keys of each query tile cut into `ranges` parts over the chip, for few rows over a
+ * long cache: fp32 partials in ws (16-byte aligned, the bytes afx_prefill_attn_plan gives for its own count), a
+ * second launch merges them. */
+int afx_prefill_attn_split(const void* q, int ldq, const void* kcache, const void* vcache, long long kv_hs, int Mmax,
+                           void* o, int ldo, int M, int pos0, int Hq, int Hkv, int D, float scale, int ranges, void* ws,
+                           long long ws_bytes, void* stream);
+/* The ranges worth cutting at this shape (1: use afx_prefill_attn) and, optionally, their workspace. */
+int afx_prefill_attn_plan(int M, int pos0, int Hq, int Hkv, int D, long long* ws_bytes);
 
 #ifdef __cplusplus
 }

@@ -256,3 +256,37 @@ def test_gemm_epilogues_every_form(fmt, M, N, K, epi):
         check_f16(outs[0], ref.r16(ref.silu(g) * u), what=f"gemm {fmt} swiglu")
     else:
         check_f16(outs[0], lin, what=f"gemm {fmt} f32")
+
+
+@pytest.mark.parametrize("M,pos0,Hq,Hkv,Mmax", [(1, 5, 4, 2, 64), (7, 300, 16, 8, 320), (64, 64, 8, 2, 200), (130, 500, 8, 8, 700),
+                                                (129, 0, 4, 4, 129)])
+def test_prefill_attention_split_keys(M, pos0, Hq, Hkv, Mmax):
+    """The keys of each tile cut into ranges (one, some, more than there are key blocks: empty ranges, and
+    ranges wholly past a query's position): the oracle's bar, and the same fp32 arithmetic as form 3 up to
+    the order of the sums and the fp16 probabilities' scale (two fp16 ulps of the largest value)."""
+    import torch
+    from aneforge_amd import _kernels as Kn
+    D = 128
+    rng = np.random.default_rng(M + pos0)
+    L = pos0 + M
+    Kc, Vc = (rng.standard_normal((Hkv, Mmax, D)).astype(np.float16) for _ in range(2))
+    Kc[:, L:], Vc[:, L:] = 60000.0, 60000.0
+    q = rng.standard_normal((M, Hq * D)).astype(np.float16)
+    mask = np.where(np.arange(L)[None, :] <= pos0 + np.arange(M)[:, None], 0.0, -np.inf)
+    want = ref.attention(q.reshape(M, Hq, D).transpose(1, 0, 2)[None], Kc[None, :, :L], Vc[None, :, :L], mask=mask)
+    want = want[0].transpose(1, 0, 2).reshape(M, Hq * D)
+    base = torch.zeros((M, Hq * D), dtype=torch.float16, device="cuda")
+    Kn.prefill_attn(dev(q), dev(Kc), dev(Vc), base, pos0, Hq, Hkv)
+    ulp = float(np.spacing(np.float16(np.abs(want).max())))
+    for ranges in (1, 2, 5, 16):
+        say(f"prefill_attn_split ranges={ranges} M={M} pos0={pos0} Hq={Hq} Hkv={Hkv}")
+        ws = torch.full((ranges * M * Hq * (D + 2),), float("nan"), dtype=torch.float32, device="cuda")
+        o = torch.zeros_like(base)
+        Kn.prefill_attn_split(dev(q), dev(Kc), dev(Vc), o, pos0, Hq, Hkv, ranges, ws)
+        check_f16(host(o), want, what=f"prefill attention, {ranges} key ranges")
+        assert np.abs(host(o).astype(np.float64) - host(base).astype(np.float64)).max() <= 2 * ulp
+    with pytest.raises(RuntimeError, match="workspace"):
+        Kn.prefill_attn_split(dev(q), dev(Kc), dev(Vc), o, pos0, Hq, Hkv, 16, ws[:8])
+    r, nbytes = Kn.prefill_attn_plan(M, pos0, Hq, Hkv, D)
+    assert r >= 1 and (nbytes == r * M * Hq * (D + 2) * 4 if r > 1 else nbytes == 0)
+    assert Kn.prefill_attn_plan(100, 2048, 32, 8, D)[0] > 1 and Kn.prefill_attn_plan(2048, 0, 32, 8, D)[0] == 1
