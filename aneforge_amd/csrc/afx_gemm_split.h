@@ -41,6 +41,7 @@ struct SplitArgs {
   int T, E, topk, x_by_token;   // MoE: tokens, experts, top-k, X row of an entry = entry / topk or the entry
   int ldx, ldy, M, N, K, epi;
   int S, tiles_n, tiles_m, mt, nw; // slices and tiles (MoE: one slice; row tiles are found from cnt)
+  int rp;                  // rows of a 16-row tile kept in the workspace (M below 16 rows, else 16)
   int xbytes;              // bytes of X the loads may read (< 2^31)
   int vec;                 // y (and resid, bias) rows take 4-element accesses
 };
@@ -465,10 +466,11 @@ __global__ __launch_bounds__(512, 2) void gemm_split_kernel(SplitArgs a) {
       float v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = acc[m][j][i] * sc[i];
-      if (a.S > 1)
-        *(f4*)(a.ws + ((((size_t)slice * a.tiles_m * a.tiles_n + tile) * (NW * NT) + wn * NT + j) * MT + m) * 256 + lane * 4) =
-            (f4){v[0], v[1], v[2], v[3]};
-      else if (mr < rows) split_store4(a, v, n, lst ? lst[mr] : mr);
+      if (a.S > 1) {
+        if (r < a.rp)
+          ((f4*)a.ws)[(((((size_t)slice * a.tiles_m * a.tiles_n + tile) * (NW * NT) + wn * NT + j) * MT + m) * 4 + g) * a.rp + r] =
+              (f4){v[0], v[1], v[2], v[3]};
+      } else if (mr < rows) split_store4(a, v, n, lst ? lst[mr] : mr);
     }
   }
 }
@@ -505,6 +507,8 @@ struct SplitPlan {
   float us;                // its predicted time
 };
 bool split_supported(int fmt, int N, int K);
+// afx_gemm_split's launches, `a` filled in but for the plan's fields; w, x and ws 16-byte aligned.
+int split_launch(int fmt, SplitArgs& a, long long ws_bytes, hipStream_t stream, const char* what);
 SplitPlan split_plan(int fmt, int M, int N, int K);
 // The grouped experts (a.cnt set): a's pointers, strides, T, E, topk, N, K and epi filled in by the caller.
 int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what);

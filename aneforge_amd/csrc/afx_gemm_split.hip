@@ -87,8 +87,9 @@ static float gemm_tile_us(int fmt, int M, int N, int K) {
   }
   return (float)us;
 }
-static long long split_ws_bytes(const SplitPlan& p, int S) {
-  return (long long)S * p.tiles_m * p.tiles_n * p.mt * p.nw * 2048;
+static int split_rows_kept(int M) { return M < 16 ? M : 16; }
+static long long split_ws_bytes(const SplitPlan& p, int M, int S) {
+  return (long long)S * p.tiles_m * p.tiles_n * p.mt * p.nw * 128 * split_rows_kept(M);
 }
 
 // y = epilogue(sum of the S slices of ws in slice order), four output features of one row per thread;
@@ -96,11 +97,12 @@ static long long split_ws_bytes(const SplitPlan& p, int S) {
 __global__ __launch_bounds__(256) void gemm_split_finish_kernel(SplitArgs a) {
   const int nt = 2 * a.nw;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long per = (long long)a.tiles_m * a.tiles_n * nt * a.mt * 64;   // f4 per slice
+  const long long per = (long long)a.tiles_m * a.tiles_n * nt * a.mt * 4 * a.rp;   // f4 per slice
   if (idx >= per) return;
-  const int lane = (int)(idx & 63), q0 = (int)(idx >> 6), q1 = q0 / a.mt, tile = q1 / nt;
-  const int n = (tile / a.tiles_m) * (16 * nt) + 16 * (q1 % nt) + 4 * (lane >> 4);
-  const int m = ((tile % a.tiles_m) * a.mt + q0 % a.mt) * 16 + (lane & 15);
+  const int gr = (int)(idx / a.rp), r = (int)(idx - (long long)gr * a.rp);
+  const int q0 = gr >> 2, q1 = q0 / a.mt, tile = q1 / nt;
+  const int n = (tile / a.tiles_m) * (16 * nt) + 16 * (q1 % nt) + 4 * (gr & 3);
+  const int m = ((tile % a.tiles_m) * a.mt + q0 % a.mt) * 16 + r;
   if (n >= a.N || m >= a.M) return;
   const f4* w = (const f4*)a.ws + idx;
   float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -130,8 +132,9 @@ static split_fn pick(int fmt, int mt, int nw) {
   }
 }
 
-// Experts: the row tile covers about 1.25 times the mean tokens of an expert (a longer list takes several
-// tiles); the grid holds the most row tiles T * topk entries can make.
+// Experts: the row tile covers about 1.25 times the mean tokens of an expert, up to 96 rows, two workgroups
+// per CU (a longer list takes several tiles: 1024 tokens of top-2 over 8 Q4_0 experts take 657 + 310 us in
+// them, 755 + 369 in 128-row tiles); the grid holds the most row tiles T * topk entries can make.
 int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what) {
   AFX_REQUIRE(a.w && a.x && a.y && a.cnt && a.list, "%s: null pointer", what);
   AFX_REQUIRE(a.T >= 1 && a.topk >= 1 && a.E >= 1 && split_supported(fmt, a.N, a.K), "%s: bad sizes", what);
@@ -143,8 +146,15 @@ int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what
   AFX_REQUIRE(xbytes < 0x7fff0000LL, "%s: activations span %lld bytes (limit 2 GiB)", what, xbytes);
   a.xbytes = (int)xbytes;
   const double mean = 1.25 * entries / a.E / 16;   // in 16-row tiles
-  const int mt = mean <= 1 ? 1 : mean <= 2 ? 2 : mean <= 3 ? 3 : mean <= 4 ? 4 : mean <= 6 ? 6 : 8;
-  const int nw = (double)((a.N + 127) / 128) * (a.E < entries ? a.E : entries) >= 256 ? 4 : 2;
+  int mt = mean <= 1 ? 1 : mean <= 2 ? 2 : mean <= 3 ? 3 : mean <= 4 ? 4 : 6;
+  int nw = (double)((a.N + 127) / 128) * (a.E < entries ? a.E : entries) >= 256 ? 4 : 2;
+  const char* es = getenv("AFX_GEMM_SPLIT");       // as split_plan's (the slice count does not apply)
+  int fs = 0, fn = 0, fm = 0;
+  if (es && sscanf(es, "%d.%d.%d", &fs, &fn, &fm) >= 2) {
+    if (fn == 2 || fn == 4 || fn == 8) nw = fn;
+    if (fm >= 1) mt = fm <= 4 ? fm : fm <= 6 ? 6 : 8;
+    if (!split_built(fmt, mt, nw)) nw = 4;
+  }
   a.S = 1; a.M = 0; a.mt = mt; a.nw = nw;
   a.tiles_n = (a.N + 32 * nw - 1) / (32 * nw);
   const long long tiles = entries / (16 * mt) + (a.E < entries ? a.E : entries);
@@ -152,6 +162,29 @@ int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what
   const bool glu = a.epi == EPI_SWIGLU || a.epi == EPI_GEGLU;
   a.vec = glu ? a.ldy % 2 == 0 && ((uintptr_t)a.y & 3) == 0 : a.ldy % 4 == 0 && ((uintptr_t)a.y & 15) == 0;
   hipLaunchKernelGGL(pick(fmt, mt, nw), dim3((unsigned)(tiles * a.tiles_n)), dim3(512), 0, stream, a);
+  return check_launch(what);
+}
+
+int split_launch(int fmt, SplitArgs& a, long long ws_bytes, hipStream_t stream, const char* what) {
+  const SplitPlan p = split_plan(fmt, a.M, a.N, a.K);
+  a.S = p.S;
+  while (a.S > 1 && (!a.ws || split_ws_bytes(p, a.M, a.S) > ws_bytes)) --a.S;
+  a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.mt = p.mt; a.nw = p.nw;
+  a.rp = split_rows_kept(a.M);
+  const bool glu = a.epi == EPI_SWIGLU || a.epi == EPI_GEGLU;
+  a.vec = a.epi == EPI_F32 ? a.ldy % 4 == 0 && ((uintptr_t)a.y & 15) == 0
+        : glu ? a.ldy % 2 == 0 && ((uintptr_t)a.y & 3) == 0
+        : a.ldy % 4 == 0 && ((uintptr_t)a.y & 7) == 0 && (a.epi != EPI_RESID || ((uintptr_t)a.resid & 7) == 0);
+  const long long xbytes = ((long long)(a.M - 1) * a.ldx + a.K) * 2;
+  AFX_REQUIRE(xbytes < (1ll << 31), "%s: activations span %lld bytes (limit 2 GiB)", what, xbytes);
+  a.xbytes = (int)xbytes;
+  const long long blocks = ((long long)a.tiles_n * a.S + 7) / 8 * 8 * a.tiles_m;
+  AFX_REQUIRE(blocks < (1ll << 31), "%s: %lld tiles", what, blocks);
+  hipLaunchKernelGGL(pick(fmt, p.mt, p.nw), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  const int rc = check_launch(what);
+  if (rc || a.S == 1) return rc;
+  const long long n = split_ws_bytes(p, a.M, 1) / 16;
+  hipLaunchKernelGGL(gemm_split_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
   return check_launch(what);
 }
 
@@ -165,7 +198,7 @@ int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes) {
   if (ws_bytes) *ws_bytes = 0;
   AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K), "afx_gemm_split_plan: fmt=%d M=%d N=%d K=%d is not afx_gemm_split's", fmt, M, N, K);
   const SplitPlan p = split_plan(fmt, M, N, K);
-  if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, p.S) : 0;
+  if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, M, p.S) : 0;
   return p.us < 0.88f * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
 }
 
@@ -177,8 +210,6 @@ int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int
               "afx_gemm_split: need M >= 1, N %% 16 == 0, K %% 128 == 0 (256 for K-quants) (fmt=%d M=%d N=%d K=%d)", fmt, M, N, K);
   AFX_REQUIRE(ldx >= K && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0,
               "afx_gemm_split: x and weights must be 16-byte aligned rows (ldx %% 8 == 0)");
-  const long long xbytes = ((long long)(M - 1) * ldx + K) * 2;
-  AFX_REQUIRE(xbytes < (1ll << 31), "afx_gemm_split: activations span %lld bytes (limit 2 GiB)", xbytes);
   AFX_REQUIRE((epi >= 0 && epi <= 3) || epi == EPI_GEGLU, "afx_gemm_split: unknown epilogue %d", epi);
   AFX_REQUIRE(fmt == FMT_F16 || scale, "afx_gemm_split: quantized weights need scales");
   const int align = fmt == FMT_L4 ? 15 : fmt == FMT_Q4 || fmt == FMT_BW ? 7 : fmt == FMT_Q4K || fmt == FMT_Q6K ? 3 : 1;
@@ -191,22 +222,7 @@ int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int
   a.w = w; a.scale = (const half_t*)scale; a.bias = (const half_t*)bias; a.x = (const half_t*)x; a.y = y;
   a.resid = (const half_t*)residual; a.ldx = ldx; a.ldy = ldy; a.M = M; a.N = N; a.K = K; a.epi = epi;
   a.ws = (float*)ws;
-  a.xbytes = (int)xbytes;
-  const SplitPlan p = split_plan(fmt, M, N, K);
-  a.S = p.S;
-  while (a.S > 1 && (!ws || split_ws_bytes(p, a.S) > ws_bytes)) --a.S;
-  a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.mt = p.mt; a.nw = p.nw;
-  a.vec = epi == EPI_F32 ? ldy % 4 == 0 && ((uintptr_t)y & 15) == 0
-        : glu ? ldy % 2 == 0 && ((uintptr_t)y & 3) == 0
-        : ldy % 4 == 0 && ((uintptr_t)y & 7) == 0 && (epi != EPI_RESID || ((uintptr_t)residual & 7) == 0);
-  const long long blocks = ((long long)a.tiles_n * a.S + 7) / 8 * 8 * a.tiles_m;
-  AFX_REQUIRE(blocks < (1ll << 31), "afx_gemm_split: %lld tiles", blocks);
-  hipLaunchKernelGGL(pick(fmt, p.mt, p.nw), dim3((unsigned)blocks), dim3(512), 0, (hipStream_t)stream, a);
-  int rc = check_launch("afx_gemm_split");
-  if (rc || a.S == 1) return rc;
-  const long long n = split_ws_bytes(p, 1) / 16;
-  hipLaunchKernelGGL(gemm_split_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a);
-  return check_launch("afx_gemm_split(finish)");
+  return split_launch(fmt, a, ws_bytes, (hipStream_t)stream, "afx_gemm_split");
 }
 
 }  // extern "C"

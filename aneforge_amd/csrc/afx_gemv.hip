@@ -2,6 +2,7 @@
 // Host-side validation happens here, before any launch, so a bad call returns an error code
 // instead of reaching a kernel with extents it does not expect.
 #include <stdlib.h>
+#include "afx_gemm_split.h"
 #include "afx_gemv_impl.h"
 #include "afx_mfma.h"
 
@@ -88,9 +89,25 @@ static int launch(int fmt, GemvArgs& a, int eg, int rows_hint, hipStream_t strea
     AFX_REQUIRE(a.dh >= 2 && a.dh % 2 == 0 && a.nq % a.dh == 0 && a.nk % a.dh == 0 && a.pos && a.kcache &&
                     a.vcache,
                 "%s: bad fused-QKV arguments", what);
-  // 4+ activation rows without a norm prologue: the dot products go to MFMA (any row count, in
-  // groups of 16); the vector kernels below take at most 8 rows
-  if (a.M >= mfma_min_rows() && eg != EG_QKV && !a.gamma && mfma_supported(fmt, a.K) && a.N % 4 == 0) {
+  // The int4 codebook and the K-quants have no skinny MFMA kernel, and fp16 rows past 4096 leave that
+  // kernel's registers: the split GEMM (afx_gemm_split.h) takes them, with the caller's workspace for
+  // its K slices.  From 5 rows, where the vector kernels take 8 (Q4_K 22016 x 4096 at 8 rows 157 -> 33
+  // us, 2048 x 2048 12 -> 8.4), and from 3 on large matrices (46.6 -> 33; 4096 x 4096 is even there).
+  const long long weights = (long long)a.N * a.K;
+  const bool split_fmt = fmt == FMT_L4 || fmt == FMT_Q4K || fmt == FMT_Q6K || (fmt == FMT_F16 && a.K > 4096);
+  if (split_fmt && mfma_min_rows() <= 4 && eg != EG_QKV && !a.gamma && a.M >= (fmt == FMT_F16 || weights >= 40000000 ? 3 : 5) &&
+      split_supported(fmt, a.N, a.K) && (!a.ws || ((uintptr_t)a.ws & 15) == 0)) {
+    SplitArgs s = {};
+    s.w = a.w; s.scale = a.scale; s.x = a.x; s.ldx = a.ldx; s.y = a.y; s.ldy = a.ldy; s.bias = a.bias; s.resid = a.resid;
+    s.ws = a.ws; s.M = a.M; s.N = a.N; s.K = a.K; s.epi = a.epi;
+    return split_launch(fmt, s, a.ws_bytes, stream, what);
+  }
+  // 4+ activation rows without a norm prologue: the dot products go to MFMA (any row count, in groups of
+  // 16); the vector kernels below take at most 8 rows.  3 rows too on packed matrices of 8 M weights or
+  // more whose rows the persistent kernel takes, where the vector kernel's padded fourth row costs more
+  // (int8 22016 x 4096 42.5 -> 20 us, Q4_0 4096 x 4096 11.1 -> 6.5; fp16 is even).
+  const bool three = mfma_min_rows() == 4 && weights >= 8000000 && fmt != FMT_F16 && (fmt == FMT_Q4 || a.K <= 4096 || a.ws);
+  if (a.M >= (three ? 3 : mfma_min_rows()) && eg != EG_QKV && !a.gamma && mfma_supported(fmt, a.K) && a.N % 4 == 0) {
     MfmaArgs m = {};
     m.w = a.w; m.scale = a.scale; m.x = a.x; m.ldx = a.ldx; m.y = a.y; m.ldy = a.ldy;
     m.bias = a.bias; m.resid = a.resid; m.M = a.M; m.N = a.N; m.K = a.K; m.epi = a.epi;
