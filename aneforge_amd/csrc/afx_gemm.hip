@@ -81,14 +81,22 @@ __device__ __forceinline__ h8 i8x8_to_h8(u2 v) {
 // freed staging registers (so global loads still get a full step); one barrier publishes the stage;
 // and the next step's first fragments are read between the second half-step's products.  No LDS read
 // then waits at the top of a step, which pays where a CU holds a single workgroup (tiles <= CUs).
+// 7 (fp16 weights): form 6's order over a 256 x 256 tile, eight wavefronts of 128 x 64.  A product of
+// 16 x 16 needs 12 fragment reads per 32 instead of 6 per 8, and a tile half the L2 traffic per product,
+// at one workgroup per CU (128 KB of LDS).  For int8 codes the conversion beside the products, which two
+// wavefronts per SIMD no longer hide, costs more than that gives (22016 x 4096 at M = 2048: 417 us,
+// form 3 367; a 256 x 128 tile 454), so it is built for fp16 only.
 // (The same order over form 3's layout, "form 5", needed 168 VGPRs with spills and measured even with
 // form 3; it is not instantiated.)
 template <int WL> struct WaveLayout {
-  static constexpr bool W8 = WL == 4 || WL == 6;     // eight wavefronts in 2 x 4
+  static constexpr bool W8 = WL == 4 || WL >= 6;     // eight wavefronts in 2 x 4
   static constexpr bool Q4 = WL == 0;                // four wavefronts in 2 x 2
-  static constexpr int MT = W8 ? 4 : (Q4 ? 4 : 8), NT = W8 ? 2 : (Q4 ? 4 : 2);
+  static constexpr int WN = Q4 ? 2 : 4;             // wavefronts side by side in N
+  static constexpr int MT = WL == 7 ? 8 : W8 || Q4 ? 4 : 8, NT = WL == 7 || Q4 ? 4 : 2;
   static constexpr int NTH = W8 ? 512 : 256;        // threads per workgroup
-  static constexpr int WPE = W8 ? 4 : 3;            // wavefronts per SIMD the register budget is sized for
+  static constexpr int WPE = WL == 7 ? 2 : W8 ? 4 : 3;   // wavefronts per SIMD the register budget is sized for
+  static constexpr int BM = WL == 7 ? 256 : kGBM, BN = WL == 7 ? 256 : kGBN;
+  static_assert(BM == MT * 16 * (NTH / 64 / WN) && BN == NT * 16 * WN, "the wavefronts cover the tile");
 };
 template <int V> struct Stage { static constexpr int value = V; };
 
@@ -133,11 +141,13 @@ template <int FMT, int EG, int WL>
 __global__ __launch_bounds__(WaveLayout<WL>::NTH)
 __attribute__((amdgpu_waves_per_eu(WaveLayout<WL>::WPE, WaveLayout<WL>::WPE))) void gemm_kernel(GemmArgs a) {
   constexpr int MT = WaveLayout<WL>::MT, NT = WaveLayout<WL>::NT, NTH = WaveLayout<WL>::NTH;
-  constexpr int WS = GemmW<FMT>::kStride, WR = GemmW<FMT>::kRow, WC = GemmW<FMT>::kChunks * 256 / NTH;
-  constexpr int AC = 4 * 256 / NTH;                 // 16-byte activation chunks per thread and stage
+  constexpr int BM = WaveLayout<WL>::BM, BN = WaveLayout<WL>::BN;
+  constexpr int WS = GemmW<FMT>::kStride, WR = GemmW<FMT>::kRow, WC = BN * (WR / 16) / NTH;
+  constexpr int AC = BM * 8 / NTH;                  // 16-byte activation chunks per thread and stage
+  static_assert(FMT != FMT_BW || BN == kGBN, "one block-scale thread per weight row");
   constexpr bool kCodes = FMT == FMT_I8 || FMT == FMT_BW;   // one byte per weight
-  __shared__ __align__(16) unsigned char As[2][kGBM * kGAStride];
-  __shared__ __align__(16) unsigned char Bs[2][kGBN * WS];
+  __shared__ __align__(16) unsigned char As[2][BM * kGAStride];
+  __shared__ __align__(16) unsigned char Bs[2][BN * WS];
   __shared__ uint32_t Ss[2][FMT == FMT_BW ? kGBN : 1];    // blockwise: the 2 block scales of each row's step
   const int id = blockIdx.x;
   int n0, m0;
@@ -151,18 +161,18 @@ __attribute__((amdgpu_waves_per_eu(WaveLayout<WL>::WPE, WaveLayout<WL>::WPE))) v
     const int span = a.gn * a.tiles_m;
     const int g = l / span, r = l - g * span;
     const int gs = ne - nb - g * a.gn < a.gn ? ne - nb - g * a.gn : a.gn;
-    n0 = (nb + g * a.gn + r % gs) * kGBN;
-    m0 = (r / gs) * kGBM;
+    n0 = (nb + g * a.gn + r % gs) * BN;
+    m0 = (r / gs) * BM;
   } else {
     // tile: the XCD (id % 8) gets a contiguous range of logical tiles, row tiles fastest
     const int logical = (id & 7) * a.per_xcd + (id >> 3);
     if (logical >= a.tiles) return;                 // whole workgroup: no barrier reached
-    n0 = (logical / a.tiles_m) * kGBN;
-    m0 = (logical % a.tiles_m) * kGBM;
+    n0 = (logical / a.tiles_m) * BN;
+    m0 = (logical % a.tiles_m) * BM;
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr bool W8 = WaveLayout<WL>::W8, Q4 = WaveLayout<WL>::Q4;
-  const int wm = W8 ? wave >> 2 : (Q4 ? wave >> 1 : 0), wn = W8 ? wave & 3 : (Q4 ? wave & 1 : wave);
+  constexpr int WN = WaveLayout<WL>::WN;
+  const int wm = wave / WN, wn = wave % WN;
   const int M = a.M, N = a.N, K = a.K;
   const int nk = K / kGBK;
 
@@ -245,7 +255,7 @@ __attribute__((amdgpu_waves_per_eu(WaveLayout<WL>::WPE, WaveLayout<WL>::WPE))) v
 
   load(0);
   stage(0);
-  if constexpr (WL == 6) {
+  if constexpr (WL >= 6) {
     if (nk > 1) load(1);                           // the mid-step form keeps one step of loads in flight
   }
   __syncthreads();
@@ -337,7 +347,7 @@ __attribute__((amdgpu_waves_per_eu(WaveLayout<WL>::WPE, WaveLayout<WL>::WPE))) v
     if (kt + 1 < nk) stage(s ^ 1);                 // the other stage was last read before the previous barrier
     __syncthreads();
   };
-  if constexpr (WL == 6) {
+  if constexpr (WL >= 6) {
     typedef typename std::conditional<kCodes, u2, u4>::type Raw;
     auto read_a = [&](int s, int kk, int i) {
       return __builtin_bit_cast(h8, *(const u4*)(As[s] + swz16(wm * MT * 16 + i * 16 + fr, kk * 4 + fg)));
@@ -448,16 +458,14 @@ int afx_gemm(int fmt, const void* w, const void* scale, const void* x, int ldx, 
   a.w = w; a.scale = (const half_t*)scale; a.bias = (const half_t*)bias; a.x = (const half_t*)x; a.y = y;
   a.resid = (const half_t*)residual; a.ldx = ldx; a.ldy = ldy; a.M = M; a.N = N; a.K = K; a.epi = epi;
   a.tiles_m = (M + kGBM - 1) / kGBM;
-  a.tiles = a.tiles_m * ((N + kGBN - 1) / kGBN);
-  a.per_xcd = (a.tiles + 7) / 8;
   a.tiles_n = (N + kGBN - 1) / kGBN;
+  a.tiles = a.tiles_m * a.tiles_n;
   // tile order: groups of 8 weight tiles per XCD (AFX_GEMM_GN overrides; 0 = the row-tiles-fastest
   // contiguous order).  At M = 2048 on the 7B shapes, against the contiguous order: gate/up 900 -> 947,
   // down 798 -> 815 TFLOP/s, o-proj and QKV within noise; outputs bit-identical.
   const char* ge = getenv("AFX_GEMM_GN");            // read per call: tests compare the orders in one process
   const int gn_env = ge ? atoi(ge) : 8;
   a.gn = gn_env > 0 ? gn_env : 0;
-  if (a.gn > 0) a.per_xcd = ((a.tiles_n + 7) / 8) * a.tiles_m;   // the largest XCD range
   // kernel form (outputs are bit-identical across forms): int8 codes take form 6 when the tiles fit one
   // workgroup per CU (N = 4096 at M = 1000: o-proj 57.2 -> 53.3 us, down 130.3 -> 120.9 us against form
   // 4), form 4 when they fit two (the N = 4096 shapes at M = 2048: o-proj 95.5 -> 85.9 us, down 208.6 ->
@@ -465,7 +473,10 @@ int afx_gemm(int fmt, const void* w, const void* scale, const void* x, int ldx, 
   // 930, gate/up 966 -> 994 TFLOP/s); blockwise takes form 2 (form 3 even, form 4 slower); fp16 weights
   // take form 6 (eight wavefronts without the AGPR spill-over of the four-wavefront fp16 forms, which
   // leaves them at one or two wavefronts per SIMD: at M = 2048 against form 0, QKV 137.7 -> 125.3,
-  // gate/up 470.0 -> 422.6, down 234.8 -> 214.1 us).  AFX_GEMM_WL=0|2|3|4|6 overrides.  Forms 2-6 address
+  // gate/up 470.0 -> 422.6, down 234.8 -> 214.1 us), or form 7 where its larger tiles fill the CUs
+  // (N x K at M, form 6 -> 7: 22016 x 4096 at 2048 410 -> 378 us, at 4096 816 -> 748; 4096 x 11008 at 4096
+  // 399 -> 330, at 2048 209 -> 285; 4096 x 4096 at 4096 154 -> 130).  AFX_GEMM_WL=0|2|3|4|6|7 overrides;
+  // what a format does not have takes form 0.  Forms 2-7 address
   // X and W with 31-bit buffer offsets, so larger operands take form 0.
   static int cus = 0;
   if (cus == 0) {
@@ -475,13 +486,26 @@ int afx_gemm(int fmt, const void* w, const void* scale, const void* x, int ldx, 
   }
   const char* we = getenv("AFX_GEMM_WL");           // read per call, like AFX_GEMM_GN
   const int wl_env = we ? atoi(we) : -1;
-  const int wl = wl_env >= 0 ? wl_env : (fmt == FMT_I8 ? (a.tiles <= cus ? 6 : a.tiles <= 2 * cus ? 4 : 3) : fmt == FMT_BW ? 2 : 6);
+  // fp16's form 7: a round of 256 x 256 tiles over the CUs takes what 3.3 128 x 128 tiles per CU take in
+  // form 6 (1.95 us per K step of 64 against 0.59 us a tile), so its rounds, counted on the XCD with the
+  // most tiles, have to replace more than that.
+  const long long wgs7 = 8ll * (((N + 255) / 256 + 7) / 8) * ((M + 255) / 256);
+  const bool big = 10ll * a.tiles >= 34 * cus * ((wgs7 + cus - 1) / cus);
+  const int wl = wl_env >= 0 ? wl_env : (fmt == FMT_I8 ? (a.tiles <= cus ? 6 : a.tiles <= 2 * cus ? 4 : 3) : fmt == FMT_BW ? 2 : big ? 7 : 6);
   const long long xb = ((long long)(M - 1) * ldx + K) * 2;
   const long long wb = (long long)N * K * (fmt == FMT_F16 ? 2 : 1);
-  const bool form2 = (wl == 2 || wl == 3 || wl == 4 || wl == 6) && xb < (1ll << 31) && wb < (1ll << 31);
+  const bool form2 = (wl == 2 || wl == 3 || wl == 4 || wl == 6 || (wl == 7 && fmt == FMT_F16)) && xb < (1ll << 31) && wb < (1ll << 31);
   gemm_fn fn;
   int nth = 256;
-  if (form2 && wl == 6) {
+  if (form2 && wl == 7) {
+    a.x_bytes = (int)xb;
+    a.w_bytes = (int)wb;
+    nth = 512;
+    a.tiles_m = (M + 255) / 256;
+    a.tiles_n = (N + 255) / 256;
+    a.tiles = a.tiles_m * a.tiles_n;
+    fn = glu ? gemm_kernel<FMT_F16, EG_SWIGLU, 7> : gemm_kernel<FMT_F16, EG_PLAIN, 7>;
+  } else if (form2 && wl == 6) {
     a.x_bytes = (int)xb;
     a.w_bytes = (int)wb;
     nth = 512;
@@ -512,6 +536,8 @@ int afx_gemm(int fmt, const void* w, const void* scale, const void* x, int ldx, 
     else if (fmt == FMT_BW) fn = glu ? gemm_kernel<FMT_BW, EG_SWIGLU, 0> : gemm_kernel<FMT_BW, EG_PLAIN, 0>;
     else fn = glu ? gemm_kernel<FMT_F16, EG_SWIGLU, 0> : gemm_kernel<FMT_F16, EG_PLAIN, 0>;
   }
+  // workgroups per XCD: the largest of its ranges of weight tiles, or an eighth of the tiles
+  a.per_xcd = a.gn > 0 ? ((a.tiles_n + 7) / 8) * a.tiles_m : (a.tiles + 7) / 8;
   hipLaunchKernelGGL(fn, dim3(8 * a.per_xcd), dim3(nth), 0, (hipStream_t)stream, a);
   return check_launch("afx_gemm");
 }

@@ -209,3 +209,30 @@ def test_router_rows_past_16(K, M):
     want = x.astype(np.float64) @ W.T
     got = host(K.linear("fp16", w, None, dev(x), out_f32=True))
     assert (np.abs(got - want) <= _bound(x, W, want)).all()
+
+
+@pytest.mark.parametrize("M,N,Kd,epi", [(4000, 4096, 64, "f16"), (257, 272, 128, "resid"), (300, 2320, 192, "swiglu"),
+                                        (2000, 5504, 128, "f32")])
+def test_gemm_256_tiles(K, M, N, Kd, epi):
+    """fp16 weights over 256 x 256 tiles (AFX_GEMM_WL=7; the default where they fill the chip, as in the
+    first shape) against the 128 x 128 form: the same sums in the same order, so the same bytes, with
+    ragged rows and columns and an odd and an even number of K steps."""
+    rng = np.random.default_rng(M + N)
+    w = dev((rng.standard_normal((N, Kd)) * 0.05).astype(np.float16))
+    x = dev(rng.standard_normal((M, Kd)).astype(np.float16))
+    r = rng.standard_normal((M, N)).astype(np.float16)
+    outs, old = [], os.environ.get("AFX_GEMM_WL")
+    try:
+        for wl in (None, "6", "7"):
+            os.environ.pop("AFX_GEMM_WL", None)
+            if wl:
+                os.environ["AFX_GEMM_WL"] = wl
+            say(f"gemm 256 tiles M={M} N={N} K={Kd} {epi} WL={wl}")
+            y = dev(r) if epi == "resid" else None
+            outs.append(host(K.gemm("fp16", w, None, x, y=y, residual=y, epi=epi)))
+    finally:
+        os.environ.pop("AFX_GEMM_WL", None)
+        if old is not None:
+            os.environ["AFX_GEMM_WL"] = old
+    np.testing.assert_array_equal(outs[0], outs[1])
+    np.testing.assert_array_equal(outs[2], outs[1])
