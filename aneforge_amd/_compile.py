@@ -158,6 +158,7 @@ class _Lowering:
         self.alias = alias or {}   # node id -> id of the input node whose buffer it writes in place
         self.cache = {} if cache is None else cache   # node id -> packed weights, reused when re-lowering
         self.preset = preset or {}   # node id -> an existing buffer to keep (input ports when re-lowering)
+        self._ws, self._ws_bytes = None, 0   # the split GEMMs' workspace: the largest any step of the program wants
 
     def out(self, t: Tensor) -> torch.Tensor:
         if id(t) in self.preset:
@@ -354,12 +355,19 @@ class _Lowering:
 
     def _gemv_rows(self, lin: "E.Linear", x2, y2, bias=None):
         """y2[M, N] = x2[M, K] @ W^T (+bias) as one contraction over all M rows, as the reference emits
-        one matmul for any M (aneforge/_compile.py:375-385).  Up to 16 rows: one afx_linear (vector GEMV
-        to 3 rows, the skinny MFMA kernel from 4).  From 17 rows: the MFMA GEMM, which streams the weight
-        once per 128-row tile; formats it does not read packed are expanded to fp16 first (once per
-        call, into a buffer of this program), as the batched prefill does."""
+        one matmul for any M (aneforge/_compile.py:375-385).  Up to 16 rows: one afx_linear.  From 17 rows:
+        the split GEMM where its plan is the faster (every packed format; its partials go to a workspace
+        of this program, which its steps reuse in stream order), else the MFMA GEMM, on int8 and fp16
+        weights as they are and on the others' fp16 expansion (once per call, into a buffer of this
+        program), as the batched prefill does."""
         M = x2.shape[0]
         if M >= self._GEMM_MIN_ROWS and lin.K % 64 == 0 and lin.N % 16 == 0:
+            split, ws_bytes = E.gemm_plan(lin.fmt, M, lin.N, lin.K)
+            if split:
+                self._ws_bytes = max(self._ws_bytes, ws_bytes)
+                self.steps.append(lambda: K.gemm_split(lin.fmt, lin.w, lin.scale, x2, y2, bias=bias,
+                                                       ws=self._ws))
+                return
             if lin.fmt in E._GEMM_FMTS:
                 self.steps.append(lambda: K.gemm(lin.fmt, lin.w, lin.scale, x2, y=y2, bias=bias))
                 return
@@ -568,6 +576,8 @@ def _build(outs, compress, compress_atol, block_size):
         preset = {id(t): keep[t._name] for t in inputs} if keep else None
         low = _Lowering(compress, compress_atol, block_size, alias, cache, preset)
         low.lower(order)
+        if low._ws_bytes:
+            low._ws = torch.empty(low._ws_bytes // 4, dtype=torch.float32, device="cuda")
         bufs = {t._name: low.buf[id(t)] for t in inputs}
         for o in outs:
             bufs[o._name] = low.buf[id(o)]

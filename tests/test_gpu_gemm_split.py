@@ -236,3 +236,34 @@ def test_gemm_256_tiles(K, M, N, Kd, epi):
             os.environ["AFX_GEMM_WL"] = old
     np.testing.assert_array_equal(outs[0], outs[1])
     np.testing.assert_array_equal(outs[2], outs[1])
+
+
+@pytest.mark.parametrize("compress", [None, "int8", "int4", "blockwise"])
+@pytest.mark.parametrize("rows", [17, 64])
+def test_compiled_matmul_rows(compress, rows):
+    """A compiled graph's matmuls of 17 and 64 rows, two of them sharing the program's workspace, against
+    the same matmuls row by row in batches of 16 (the linear kernels): both within their own rounding of
+    the fp64 product, so within two fp16 ulps and the two accumulations' bound of each other."""
+    import aneforge_amd as af
+    rng = np.random.default_rng(rows)
+    D, F = 512, 2048
+    w1 = (rng.standard_normal((F, D)) / np.sqrt(D)).astype(np.float32)
+    w2 = (rng.standard_normal((D, F)) / np.sqrt(F)).astype(np.float32)
+
+    def net(n):
+        x = af.input((n, D))
+        h = x.linear(w1)
+        return af.compile(h.relu().linear(w2), compress=compress, compress_atol=1.0)
+    x = rng.standard_normal((rows, D)).astype(np.float16)
+    say(f"compiled matmul rows={rows} {compress}")
+    full = net(rows)
+    got = [np.asarray(full(x)) for _ in range(3)]
+    part = net(16)
+    pad = np.concatenate([x, np.zeros((-rows % 16, D), np.float16)])
+    want = np.concatenate([np.asarray(part(pad[i:i + 16])) for i in range(0, len(pad), 16)])[:rows]
+    np.testing.assert_array_equal(got[1], got[0])
+    np.testing.assert_array_equal(got[2], got[0])
+    # an intermediate that rounds the other way moves by an ulp (2^-10 relative at most) and its share of
+    # an output is a sum of such moves over F terms: sqrt(F / 2) * 2^-10 * |h| |w| at 6 deviations
+    tol = 6 * np.sqrt(F / 2) * 2.0 ** -10 * np.abs(want).std() / np.sqrt(F) * 2 + 2.0 ** -10 * np.abs(want)
+    assert (np.abs(got[0] - want) <= tol).all()
