@@ -267,3 +267,29 @@ def test_compiled_matmul_rows(compress, rows):
     # an output is a sum of such moves over F terms: sqrt(F / 2) * 2^-10 * |h| |w| at 6 deviations
     tol = 6 * np.sqrt(F / 2) * 2.0 ** -10 * np.abs(want).std() / np.sqrt(F) * 2 + 2.0 ** -10 * np.abs(want)
     assert (np.abs(got[0] - want) <= tol).all()
+
+
+def test_three_rows_with_scales_off_the_mfma_alignment(K):
+    """3 rows of a large int8 matrix take the skinny MFMA kernel only where its 8-byte scale loads do."""
+    rng = np.random.default_rng(5)
+    N, Kd = 2048, 4096
+    w, s, W = _weights(K, "int8", N, Kd, rng)
+    off = torch.empty(N + 1, dtype=torch.float16, device="cuda")[1:]
+    off.copy_(s)
+    x = rng.standard_normal((3, Kd)).astype(np.float16)
+    want = x.astype(np.float64) @ W.T
+    for sc in (s, off):
+        say(f"int8 3 rows scale at {sc.data_ptr() % 16}")
+        assert (np.abs(host(K.linear("int8", w, sc, dev(x))) - want) <= _bound(x, W, want)).all()
+
+
+def test_codebook_rows_past_the_split_range(K):
+    """Activation rows that span 2 GiB (a stride of 2^27) stay on the vector kernels, in two launches."""
+    rng = np.random.default_rng(6)
+    w, s, W = _weights(K, "lut4", 16, 256, rng)
+    x = rng.standard_normal((9, 256)).astype(np.float16)
+    wide = torch.empty((9, 1 << 27), dtype=torch.float16, device="cuda")[:, :256]
+    wide.copy_(dev(x))
+    want = x.astype(np.float64) @ W.T
+    say("lut4 9 rows, row stride 2^27")
+    assert (np.abs(host(K.linear("lut4", w, s, wide)) - want) <= _bound(x, W, want)).all()
