@@ -412,7 +412,7 @@ __global__ __launch_bounds__(512, 2) void gemm_split_kernel(SplitArgs a) {
   auto step = [&](auto b, int t, int s) {
     constexpr int B = decltype(b)::value;
     load(b, t + PD);
-    compute(s);
+    if (FMT != FMT_L4 || t < t1) compute(s);       // a zero chunk's codes would still name codebook entry 0, which may be infinite
     stage(Buf<(B + 1) % PD>{}, s ^ 1);             // last read before the previous barrier
     __syncthreads();
   };

@@ -293,3 +293,22 @@ def test_codebook_rows_past_the_split_range(K):
     want = x.astype(np.float64) @ W.T
     say("lut4 9 rows, row stride 2^27")
     assert (np.abs(host(K.linear("lut4", w, s, wide)) - want) <= _bound(x, W, want)).all()
+
+
+@pytest.mark.parametrize("slices", [1, 3])
+def test_unused_infinite_codebook_entry(K, slices, monkeypatch):
+    """Entry 0 is infinite and no weight names it: the slices' odd last chunks must not bring it in."""
+    monkeypatch.setenv("AFX_GEMM_SPLIT", f"{slices}.2.1")
+    rng = np.random.default_rng(8)
+    N, Kd = 64, 128 * 9
+    idx = rng.integers(1, 16, (N, Kd))
+    packed = (idx[:, 0::2] | (idx[:, 1::2] << 4)).astype(np.uint8)
+    cb = rng.normal(0, 0.02, (N, 16)).astype(np.float16)
+    cb[:, 0] = np.inf
+    W = np.take_along_axis(cb.astype(np.float64), idx, axis=1)
+    x = rng.standard_normal((7, Kd)).astype(np.float16)
+    want = x.astype(np.float64) @ W.T
+    say(f"lut4 infinite entry, {slices} slices")
+    y = torch.empty((7, N), dtype=torch.float16, device="cuda")
+    K.gemm_split("lut4", dev(packed), dev(cb), dev(x), y, ws=torch.empty(1 << 16, dtype=torch.float32, device="cuda"))
+    assert (np.abs(host(y) - want) <= _bound(x, W, want)).all()
