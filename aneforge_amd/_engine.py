@@ -242,6 +242,14 @@ def gemm_plan(fmt: str, M: int, N: int, Kd: int):
     return K.gemm_split_plan(fmt, M, N, Kd)
 
 
+def split_plan(lin: "Linear", M: int):
+    """gemm_plan for M rows of lin; weights or scales on odd addresses (views of a caller's own packing)
+    stay on the kernels that take them."""
+    if lin.w.data_ptr() % 16 or (lin.scale is not None and lin.scale.data_ptr() % 16):
+        return False, 0
+    return gemm_plan(lin.fmt, M, lin.N, lin.K)
+
+
 @functools.lru_cache(maxsize=4096)
 def attn_plan(M: int, pos0: int, H: int, KV: int, dh: int):
     """(key ranges, workspace bytes) of the prompt rows' attention: see K.prefill_attn_plan."""
@@ -254,7 +262,7 @@ def prefill_gemm(eng, lin: "Linear", x, y, residual=None, epi="f16"):
     formats).  Otherwise afx_gemm on the packed weights (int8, fp16), or on the fp16 expansion of the
     others in the engine's weight scratch (for blockwise that measured faster than scaling the codes
     inside the GEMM: 40.7 vs 48.2 ms for the 2048-token cfg3 prompt)."""
-    split, ws_bytes = gemm_plan(lin.fmt, x.shape[0], lin.N, lin.K)
+    split, ws_bytes = split_plan(lin, x.shape[0])
     if split:
         return K.gemm_split(lin.fmt, lin.w, lin.scale, x, y, bias=lin.bias, residual=residual, epi=epi,
                             ws=eng.gemm_scratch(ws_bytes) if ws_bytes else None)
@@ -631,10 +639,14 @@ class DecodeEngine:
 
     def gemm_scratch(self, nbytes: int) -> torch.Tensor:
         """An fp32 workspace of at least nbytes for the split GEMM's and the split attention's partials
-        (reused by every launch in stream order; a prompt's largest is a few MB per hundred rows)."""
-        if getattr(self, "_gws", None) is None or self._gws.numel() * 4 < nbytes:
-            self._gws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device="cuda")
-        return self._gws
+        (reused by every launch in stream order; a prompt's largest is a few MB per hundred rows).  It at
+        least doubles when it grows, and the outgrown ones (together no larger than it) are kept: a launch
+        on another stream or a captured one may still use them."""
+        held = self.__dict__.setdefault("_gws", [])
+        if not held or held[-1].numel() * 4 < nbytes:
+            held.append(torch.empty(max((nbytes + 3) // 4, 2 * held[-1].numel() if held else 0), dtype=torch.float32,
+                                    device="cuda"))
+        return held[-1]
 
     def _prefill_buffers(self, C: int) -> dict:
         if getattr(self, "_pf", None) is None or self._pf["x"].shape[0] < C:

@@ -199,7 +199,8 @@ int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes) {
   AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K), "afx_gemm_split_plan: fmt=%d M=%d N=%d K=%d is not afx_gemm_split's", fmt, M, N, K);
   const SplitPlan p = split_plan(fmt, M, N, K);
   if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, M, p.S) : 0;
-  return p.us < 0.88f * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
+  // rows of up to 2 K elements apart stay inside the kernel's 2 GiB activation range
+  return (long long)M * K < (1ll << 29) && p.us < 0.88f * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
 }
 
 int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int ldx, void* y, int ldy, int M, int N,
@@ -212,7 +213,7 @@ int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int
               "afx_gemm_split: x and weights must be 16-byte aligned rows (ldx %% 8 == 0)");
   AFX_REQUIRE((epi >= 0 && epi <= 3) || epi == EPI_GEGLU, "afx_gemm_split: unknown epilogue %d", epi);
   AFX_REQUIRE(fmt == FMT_F16 || scale, "afx_gemm_split: quantized weights need scales");
-  const int align = fmt == FMT_L4 ? 15 : fmt == FMT_Q4 || fmt == FMT_BW ? 7 : fmt == FMT_Q4K || fmt == FMT_Q6K ? 3 : 1;
+  const int align = fmt == FMT_L4 ? 15 : fmt == FMT_I8 || fmt == FMT_F16 ? 1 : 3;
   AFX_REQUIRE(((uintptr_t)scale & align) == 0, "afx_gemm_split: scales must be %d-byte aligned", align + 1);
   AFX_REQUIRE(epi != EPI_RESID || residual, "afx_gemm_split: residual pointer required");
   const bool glu = epi == EPI_SWIGLU || epi == EPI_GEGLU;

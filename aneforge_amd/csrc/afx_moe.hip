@@ -645,11 +645,11 @@ static long long fmt_scale_halves(int fmt, long long rows, int K) {
 
 // Expert linears on the split GEMM (afx_gemm_split.h): batches of more than 16 tokens, whose weights the
 // skinny kernels would stream once per 16 tokens of an expert, and from 4 tokens the formats without a
-// skinny MFMA kernel.  Pointers it cannot take stay on the other kernels.
-static bool moe_split_ok(int fmt, int T, int N, int K, const void* w, const void* scale, const void* x) {
+// skinny MFMA kernel.  Pointers and 2 GiB of activations (xrows rows of K) it cannot take stay on the other kernels.
+static bool moe_split_ok(int fmt, int T, long long xrows, int N, int K, const void* w, const void* scale, const void* x) {
   const uintptr_t align = fmt == FMT_L4 ? 15 : fmt == FMT_I8 ? 1 : 3;
   return T > (mfma_supported(fmt, K) ? 16 : 3) && split_supported(fmt, N, K) && w && x && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 &&
-         (fmt == FMT_F16 || (scale && ((uintptr_t)scale & align) == 0));
+         (fmt == FMT_F16 || (scale && ((uintptr_t)scale & align) == 0)) && xrows * K * 2 < 0x7fff0000LL;
 }
 static int moe_split(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int N, int K,
                      const int* cnt, const int* list, void* y, int ldy, int epi, hipStream_t stream, const char* what) {
@@ -748,7 +748,7 @@ int afx_moe_topk(const float* logits, int T, int E, int k, int renorm, float* ga
 // W: [E][2F][D] gate/up interleaved rows (format fmt), x: normed hidden [T][D].
 int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int F, int D,
                    const int* cnt, const int* list, void* act, int rows_hint, void* stream) {
-  if (rows_hint == 0 && moe_split_ok(fmt, T, 2 * F, D, w, scale, x))
+  if (rows_hint == 0 && moe_split_ok(fmt, T, T, 2 * F, D, w, scale, x))
     return moe_split(fmt, w, scale, x, T, k, E, 2 * F, D, cnt, list, act, F, EPI_SWIGLU, (hipStream_t)stream, "afx_moe_gateup");
   if (rows_hint == 0 && mfma_supported(fmt, D) && F % 2 == 0) {
     MfmaArgs m = {};
@@ -772,7 +772,7 @@ int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int
 int afx_moe_down(int fmt, const void* w, const void* scale, const void* act, int T, int k, int E, int F, int D,
                  const int* cnt, const int* list, float* y, int rows_hint, void* ws, long long ws_bytes,
                  void* stream) {
-  if (rows_hint == 0 && moe_split_ok(fmt, T, D, F, w, scale, act))
+  if (rows_hint == 0 && moe_split_ok(fmt, T, (long long)T * k, D, F, w, scale, act))
     return moe_split(fmt, w, scale, act, T, k, E, D, F, cnt, list, y, D, EPI_F32, (hipStream_t)stream, "afx_moe_down");
   if (rows_hint == 0 && mfma_supported(fmt, F) && D % 4 == 0) {
     MfmaArgs m = {};
@@ -836,7 +836,7 @@ int afx_moe_down_combine(int fmt, const void* w, const void* scale, const void* 
                          const void* h, const float* gate, const void* shared, void* out, void* stream) {
   AFX_REQUIRE(h && gate && out && y, "afx_moe_down_combine: null pointer");
   int S = 1;
-  if (mfma_supported(fmt, F) && D % 4 == 0 && !moe_split_ok(fmt, T, D, F, w, scale, act)) {
+  if (mfma_supported(fmt, F) && D % 4 == 0 && !moe_split_ok(fmt, T, (long long)T * k, D, F, w, scale, act)) {
     MfmaArgs m = {};
     m.w = w; m.scale = (const half_t*)scale; m.x = (const half_t*)act; m.ldx = F; m.y = y; m.ldy = D;
     m.cnt = cnt; m.list = list; m.T = T; m.k = k; m.x_by_token = 0; m.N = D; m.K = F; m.epi = EPI_F32;

@@ -312,3 +312,17 @@ def test_unused_infinite_codebook_entry(K, slices, monkeypatch):
     y = torch.empty((7, N), dtype=torch.float16, device="cuda")
     K.gemm_split("lut4", dev(packed), dev(cb), dev(x), y, ws=torch.empty(1 << 16, dtype=torch.float32, device="cuda"))
     assert (np.abs(host(y) - want) <= _bound(x, W, want)).all()
+
+
+def test_misaligned_weights_keep_their_kernels():
+    """A plan is taken only for weights and scales on 16 bytes; the workspace keeps what it outgrew."""
+    from aneforge_amd import _engine as E
+    w = torch.zeros((4096, 4096), dtype=torch.int8, device="cuda")
+    s = torch.zeros(4097, dtype=torch.float16, device="cuda")
+    assert E.split_plan(E.Linear("int8", w, s[:4096], 4096, 4096), 64)[0]
+    assert E.split_plan(E.Linear("int8", w, s[1:], 4096, 4096), 64) == (False, 0)
+    eng = E.DecodeEngine.__new__(E.DecodeEngine)
+    a = eng.gemm_scratch(1000)
+    assert eng.gemm_scratch(500) is a
+    b = eng.gemm_scratch(1004)
+    assert b.numel() >= 2 * a.numel() and eng._gws[0] is a
