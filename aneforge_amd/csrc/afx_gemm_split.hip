@@ -17,24 +17,39 @@ bool split_supported(int fmt, int N, int K) {
   return fmt >= 0 && fmt <= 6 && N >= 16 && N % 16 == 0 && K >= kSK && K % (fmt == FMT_Q4K || fmt == FMT_Q6K ? 256 : kSK) == 0;
 }
 
+// Whether two workgroups share a CU: at most 128 registers a thread and 80 KB of LDS, as the kernels are
+// built.  Counting on two where one fits cost the row tiles of 48 to 96 rows x 128 features of these formats
+// a round of workgroups: with the right count Q4_K 22016 x 4096 at 200 rows takes 92 us for 113, blockwise
+// 11008 x 2048 at 200 rows 27 for 36, fp16 4096 x 4096 at 128 rows 15 for 19.
+static bool split_two_per_cu(int fmt, int mt, int nw) {
+  if (nw > 4 || mt > 6) return false;
+  switch (fmt) {
+    case FMT_I8: return !(mt == 3 && nw == 4);
+    case FMT_F16: case FMT_BW: case FMT_Q6K: return nw == 2 || mt <= 2;
+    case FMT_Q4K: return mt <= 2 || (nw == 2 && mt == 6);
+    default: return true;
+  }
+}
 // Microseconds of one workgroup and K chunk by row tile (16 * mt rows) and features (32 * nw), measured on
 // MI355X with int8 weights at 4096 x 4096 and 22016 x 4096; `busy` with every CU taken, where the taller
-// tiles, one workgroup per CU, slow down.  dec: what decoding a format's 128 features adds (none for int8
-// codes, two fp32 steps per weight for the K-quants; fp16: twice the bytes).
+// tiles, one workgroup per CU, slow down (not for the formats whose shorter tiles are alone on a CU too).
+// dec: what decoding a format's 128 features adds (none for int8 codes, two fp32 steps per weight for the
+// K-quants; fp16: twice the bytes).
 static float split_chunk_us(int fmt, int mt, int nw, bool busy) {
   const int i = mt <= 4 ? mt - 1 : mt <= 6 ? 4 : 5;
   static const float c4[6] = {0.35f, 0.45f, 0.53f, 0.62f, 0.74f, 0.97f};
   static const float c8[6] = {0.0f, 0.0f, 0.0f, 1.01f, 1.24f, 1.53f};
-  static const float dec[7] = {0.0f, 0.05f, 0.25f, 0.2f, 0.15f, 0.45f, 0.3f};
-  const float slow = !busy ? 1.0f : mt == 8 ? 1.2f : nw == 8 ? 1.2f : 1.0f;
+  static const float dec[7] = {0.0f, 0.05f, 0.05f, 0.1f, 0.15f, 0.45f, 0.3f};
+  const bool alone = fmt == FMT_BW || fmt == FMT_Q4K || fmt == FMT_Q6K;
+  const float slow = !busy ? 1.0f : mt == 8 && !alone ? 1.2f : nw == 8 ? 1.2f : 1.0f;
   return nw == 8 ? (c8[i] + 2.0f * dec[fmt]) * slow : (c4[i] + dec[fmt]) * slow * (nw == 4 ? 1.0f : 0.7f);
 }
 static double weight_mb(int fmt, int N, int K) {
   return (double)N * (split_row_bytes_of(fmt, K) + split_side_bytes_of(fmt, K)) * 1e-6;
 }
 
-// The tile and slice count with the least predicted time: rounds of workgroups over the CUs (two resident
-// per CU up to 192 rows x features of 32, so rounds need not be whole there) x chunks x the chunk time,
+// The tile and slice count with the least predicted time: rounds of workgroups over the CUs (rounds need
+// not be whole where two are resident per CU) x chunks x the chunk time,
 // a round's fill and drain, half of the weight stream's 5 TB/s time (the other half overlaps), and a second launch and about 0.5 us
 // per MB of partials when K is sliced.  Predictions are within 15% of what the shapes above measure at
 // 16 to 2048 rows: 4096 x 4096 at 64, 128 and 300 rows takes 13.6, 15.9 and 25.2 us where the 128 x 128
@@ -55,7 +70,7 @@ SplitPlan split_plan(int fmt, int M, int N, int K) {
       if (fn && nw != fn) continue;
       SplitPlan p = {mt, nw, (t16 + mt - 1) / mt, (N + 32 * nw - 1) / (32 * nw), 1, 0.0f};
       const double part = (double)p.tiles_m * p.tiles_n * mt * nw * 2048e-6;   // MB of one slice's partials
-      const bool two = mt <= 6 && nw <= 4 && fmt != FMT_F16;
+      const bool two = split_two_per_cu(fmt, mt, nw);
       for (int S = 1; S <= kSplitMaxS && S <= nk; ++S) {
         if (fs ? S != (fs < nk ? fs : nk) : S > 1 && nk / S < 2) continue;
         const double wgs = (double)p.tiles_m * p.tiles_n * S;
