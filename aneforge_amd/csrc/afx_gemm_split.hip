@@ -214,8 +214,12 @@ int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes) {
   AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K), "afx_gemm_split_plan: fmt=%d M=%d N=%d K=%d is not afx_gemm_split's", fmt, M, N, K);
   const SplitPlan p = split_plan(fmt, M, N, K);
   if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, M, p.S) : 0;
+  // Up to three of afx_gemm's row tiles the two predictions are taken as they are: int8 22016 x 4096 at 128
+  // rows 51 -> 43 us, 11008 x 2048 at 300 35 -> 26, and no shape more than 3% slower.  Past that the split
+  // kernel's error is the larger (int8 22016 x 4096 at 2048 rows: predicted 0.95 of afx_gemm's time, measured 1.17).
+  const float margin = M <= 384 ? 1.0f : 0.88f;
   // rows of up to 2 K elements apart stay inside the kernel's 2 GiB activation range
-  return (long long)M * K < (1ll << 29) && p.us < 0.88f * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
+  return (long long)M * K < (1ll << 29) && p.us < margin * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
 }
 
 int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int ldx, void* y, int ldy, int M, int N,

@@ -259,3 +259,12 @@ def test_sdpa_kernel_choice():
     on = _Lowering._sdpa_on_mfma
     assert on(32, 512, 512, 128) and on(4, 1500, 1500, 64) and on(8, 128, 128, 128) and on(32, 64, 64, 64)
     assert not on(8, 1, 8192, 128) and not on(4, 16, 8192, 128) and not on(32, 4, 300, 64) and not on(32, 512, 512, 96)
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd,take", [("int8", 128, 22016, 4096, True), ("int8", 300, 11008, 2048, True),
+                                             ("int8", 2048, 22016, 4096, False), ("q4_0", 64, 4096, 4096, True),
+                                             ("int8", 1 << 17, 4096, 4096, False), ("fp16", 64, 4096, 64, False)])
+def test_split_gemm_choice(fmt, M, N, Kd, take):
+    """Short prompts on the split GEMM; tall ones, 1 GiB of activations and K below its chunk are not."""
+    from aneforge_amd import _kernels as K
+    assert K.gemm_split_plan(fmt, M, N, Kd)[0] is take

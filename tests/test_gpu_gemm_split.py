@@ -326,3 +326,18 @@ def test_misaligned_weights_keep_their_kernels():
     assert eng.gemm_scratch(500) is a
     b = eng.gemm_scratch(1004)
     assert b.numel() >= 2 * a.numel() and eng._gws[0] is a
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd", [("fp16", 128, 2048, 512), ("q4_k", 100, 4096, 2816), ("blockwise", 200, 2816, 512),
+                                        ("q6_k", 512, 5632, 256), ("int8", 300, 5504, 512)])
+def test_planned_tiles(K, fmt, M, N, Kd):
+    """The plan's own tile and slices, with the workspace it asks for, on both sides of one and two workgroups per CU."""
+    rng = np.random.default_rng(M)
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    n = K.gemm_split_plan(fmt, M, N, Kd)[1]
+    want = x.astype(np.float64) @ W.T
+    say(f"planned {fmt} M={M} N={N} K={Kd} workspace {n}")
+    y = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    K.gemm_split(fmt, w, s, dev(x), y, ws=torch.empty(n // 4, dtype=torch.float32, device="cuda") if n else None)
+    assert (np.abs(host(y) - want) <= _bound(x, W, want)).all()
