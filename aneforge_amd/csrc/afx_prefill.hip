@@ -970,13 +970,21 @@ __global__ __launch_bounds__(256) void prefill_attn_merge_kernel(PrefillAttnArgs
   if (i >= rows * 32) return;
   const long long row = i >> 5;
   const int d = (int)(i & 31) * 4;
+  // The row's ranges, as the kernel above cut its tile's blocks.  One that is empty or starts past the
+  // query holds none of its keys and is left out (its accumulators may be unwritten).  A range is not told
+  // by its maximum: fmaxf drops NaN, so a range whose scores are all NaN also leaves -inf, and its NaN sum
+  // has to reach the row.
+  const int m = (int)(row % a.M), m0 = m / kPQ3 * kPQ3;
+  const int mlast = m0 + kPQ3 - 1 < a.M - 1 ? m0 + kPQ3 - 1 : a.M - 1;
+  const int nkb = (a.pos0 + mlast) / kPK + 1;
   float mx = -INFINITY;
   for (int s = 0; s < sa.S; ++s) mx = fmaxf(mx, sa.ml[2 * (s * rows + row)]);
   float l = 0.0f;
   f4 o = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int s = 0; s < sa.S; ++s) {
+    const int kb0 = nkb * s / sa.S;
+    if (kb0 == nkb * (s + 1) / sa.S || kb0 * kPK > a.pos0 + m) continue;
     const float2 p = *(const float2*)(sa.ml + 2 * (s * rows + row));
-    if (p.x == -INFINITY) continue;              // no key of the range seen
     const float w = __builtin_amdgcn_exp2f(p.x - mx);
     l += w * p.y;
     const f4 v = *(const f4*)(sa.po + (s * rows + row) * kPD + d);
@@ -984,7 +992,7 @@ __global__ __launch_bounds__(256) void prefill_attn_merge_kernel(PrefillAttnArgs
     for (int e = 0; e < 4; ++e) o[e] += w * v[e];
   }
   const float inv = 1.0f / l;
-  half_t* op = a.o + (size_t)(row % a.M) * a.ldo + (size_t)(row / a.M) * kPD + d;
+  half_t* op = a.o + (size_t)m * a.ldo + (size_t)(row / a.M) * kPD + d;
   const h2 lo = {(half_t)(o[0] * inv), (half_t)(o[1] * inv)}, hi = {(half_t)(o[2] * inv), (half_t)(o[3] * inv)};
   *(u2*)op = (u2){as_u32(lo), as_u32(hi)};
 }

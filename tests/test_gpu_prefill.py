@@ -290,3 +290,34 @@ def test_prefill_attention_split_keys(M, pos0, Hq, Hkv, Mmax):
     r, nbytes = Kn.prefill_attn_plan(M, pos0, Hq, Hkv, D)
     assert r >= 1 and (nbytes == r * M * Hq * (D + 2) * 4 if r > 1 else nbytes == 0)
     assert Kn.prefill_attn_plan(100, 2048, 32, 8, D)[0] > 1 and Kn.prefill_attn_plan(2048, 0, 32, 8, D)[0] == 1
+
+
+@pytest.mark.parametrize("M,pos0,bad", [(5, 512, 512), (5, 512, 515), (3, 300, 70), (130, 500, 628), (8, 1024, 1023)])
+def test_prefill_attention_split_keeps_nan_scores(M, pos0, bad):
+    """One NaN key row of a kv head makes every query that sees it NaN, for any number of key ranges (also
+    where it is the only key that a query sees of its range), as afx_prefill_attn does; the queries before
+    it and the other heads keep their values."""
+    import torch
+    from aneforge_amd import _kernels as Kn
+    D, Hq, Hkv = 128, 32, 8
+    rng = np.random.default_rng(bad)
+    L = pos0 + M
+    Kc, Vc = (rng.standard_normal((Hkv, L, D)).astype(np.float16) for _ in range(2))
+    Kc[3, bad, 5] = np.nan
+    q = rng.standard_normal((M, Hq * D)).astype(np.float16)
+    nan = np.zeros((M, Hq, D), bool)
+    nan[max(0, bad - pos0):, 12:16] = True                  # query heads 12..15 read kv head 3
+    base = torch.zeros((M, Hq * D), dtype=torch.float16, device="cuda")
+    Kn.prefill_attn(dev(q), dev(Kc), dev(Vc), base, pos0, Hq, Hkv)
+    assert np.array_equal(np.isnan(host(base)), nan.reshape(M, -1))
+    nkb = (L - 1) // 64 + 1
+    for ranges in (2, Kn.prefill_attn_plan(M, pos0, Hq, Hkv, D)[0], min(nkb, 64), 64):
+        say(f"prefill_attn_split NaN key {bad} ranges={ranges} M={M} pos0={pos0}")
+        ws = torch.full((ranges * M * Hq * (D + 2),), 3.0, dtype=torch.float32, device="cuda")
+        o = torch.zeros_like(base)
+        Kn.prefill_attn_split(dev(q), dev(Kc), dev(Vc), o, pos0, Hq, Hkv, ranges, ws)
+        got, want = host(o), host(base)
+        assert np.array_equal(np.isnan(got), nan.reshape(M, -1)), ranges
+        fine = ~nan.reshape(M, -1)
+        ulp = float(np.spacing(np.float16(np.abs(want[fine]).max())))   # the bar of the test above
+        assert np.abs(got[fine].astype(np.float64) - want[fine].astype(np.float64)).max() <= 2 * ulp
