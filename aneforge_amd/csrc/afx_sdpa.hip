@@ -13,9 +13,10 @@
 //    stages, merged through LDS, so the longest serial chain is half the key blocks (causal tiles are
 //    dispatched longest first).
 // V is staged row-major and read through ds_read_b64_tr_b16; a query may see no key of its half (its
-// maximum stays -inf, its weights 0).  In a block where the causal mask hides some keys from some
-// queries, a V row with an infinity or NaN would turn the hidden keys' zero weights into NaN, so such a
-// block adds its visible keys one by one.
+// maximum stays -inf, its weights 0).  A V row with an infinity or NaN would turn a hidden key's zero
+// weight into NaN, and the infinity of a visible one too (its weight's low part may be zero or negative),
+// so a block that holds one adds its visible keys one by one, each with its fp32 weight.  Looking for them
+// takes three VALU operations per two values as they are staged.
 // 32 heads (8 kv) x 512 x 128 causal: 152 -> 22 us.
 #include "afx_common.h"
 
@@ -77,21 +78,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (!in) { kr[i] = (u4){0u, 0u, 0u, 0u}; vr[i] = kr[i]; }
     }
   };
-  auto stage = [&](int s, int i4, int key0) {
+  auto stage = [&](int s, int i4) {
     uint32_t bad = 0;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
       const int c = htid + 256 * i, row = c / (D / 8), ch = c % (D / 8);
       *(u4*)(Kh + s * kKB + row * KR + ch * 16) = kr[i];
       *(u4*)(Vh + s * kVB + v_at<D>(row, ch)) = vr[i];
-      if (a.causal && key0 + kSB > wfirst - 16 * w4) {                // a block the mask can reach (uniform)
-        const uint32_t w[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
+      const uint32_t w[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t e = w[j] & 0x7C007C00u;
-          bad |= (uint32_t)((e & 0x7C00u) == 0x7C00u) | (uint32_t)((e >> 16) == 0x7C00u);
-        }
-      }
+      for (int j = 0; j < 4; ++j) bad |= ((w[j] & 0x7C007C00u) + 0x04000400u) & 0x80008000u;   // a full exponent carries into its sign
     }
     if (bad) odd[hf][i4] = 1;
   };
@@ -108,7 +104,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int d = 0; d < ND; ++d) acc[d] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
   float mrow = -INFINITY, lrow = 0.0f;
   __syncthreads();                       // odd is cleared
-  if (kb0 < kb1) stage(0, 0, kb0 * kSB);
+  if (kb0 < kb1) stage(0, 0);
   __syncthreads();
   for (int i = 0; i < trips; ++i) {
     const int kb = kb0 + i, s = i & 1, key0 = kb * kSB;
@@ -155,7 +151,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[d][e] *= alpha;
       }
-      if (!(hidden && a.causal && odd[hf][i & 3])) {
+      if (!odd[hf][i & 3]) {
         h8 hi[2], lo[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
@@ -202,7 +198,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     if (htid == 0) odd[hf][(i + 2) & 3] = 0;           // last read two blocks ago
-    if (more) stage(s ^ 1, (i + 1) & 3, key0 + kSB);   // the stage was last read before the previous barrier
+    if (more) stage(s ^ 1, (i + 1) & 3);   // the stage was last read before the previous barrier
     __syncthreads();
   }
   // the second half hands over through the idle K stages, lane-major
@@ -227,7 +223,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int d = 0; d < ND; ++d) {
     float v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = ((sa == 0.0f ? 0.0f : acc[d][e] * sa) + (sb == 0.0f ? 0.0f : xw[(d * 4 + e) * 64] * sb)) * inv;
+    for (int e = 0; e < 4; ++e) v[e] = (acc[d][e] * sa + xw[(d * 4 + e) * 64] * sb) * inv;   // a half without keys: 0 * 0
     const h2 lo = {(half_t)v[0], (half_t)v[1]}, hi = {(half_t)v[2], (half_t)v[3]};
     *(u2*)(orow + d * 16) = (u2){as_u32(lo), as_u32(hi)};
   }

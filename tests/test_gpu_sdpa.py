@@ -79,6 +79,38 @@ def test_values_hidden_by_the_causal_mask_do_not_leak(bad):
     assert (np.abs(got[:, 70:][..., rest] - want[:, 70:][..., rest]) <= np.abs(want[:, 70:][..., rest]) * 2.0 ** -11 + 4 * 2.0 ** -12).all()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal,Sq,Skv", [(False, 70, 200), (True, 150, 150), (True, 40, 300), (False, 16, 33)])
+def test_infinite_values_reach_the_queries_that_see_them(causal, Sq, Skv, D):
+    """An infinity in v gives its sign in every query that sees it (two of opposite signs, or a NaN: NaN),
+    in blocks that the mask cuts and in whole ones; as in the decode kernel."""
+    from aneforge_amd import _kernels as K
+    H, Hkv = 4, 2
+    say(f"sdpa infinite values causal={causal} Sq={Sq} Skv={Skv} D={D}")
+    rng = np.random.default_rng(Skv + D)
+    q = rng.standard_normal((H, Sq, D)).astype(np.float16)
+    k, v = (rng.standard_normal((Hkv, Skv, D)).astype(np.float16) for _ in range(2))
+    v[0, 3, 1], v[0, 20, 5], v[0, 30, 5], v[1, 5, 9], v[1, Skv - 1, 2] = np.inf, np.inf, -np.inf, np.nan, -np.inf
+    if Skv > 130:
+        v[1, 100, 40], v[0, 129, 63] = np.inf, -np.inf
+    seen = np.arange(Skv)[None] <= np.arange(Sq)[:, None] + (Skv - Sq if causal else Skv)
+    want = _want(q, k, v, D ** -0.5, causal)                # finite values only: now the others
+    for h in range(H):
+        vv = v[h * Hkv // H].astype(np.float64)
+        for key, d in zip(*np.nonzero(~np.isfinite(vv))):
+            with np.errstate(invalid="ignore"):             # inf - inf: NaN
+                want[h, seen[:, key], d] += vv[key, d]
+    got = _run(q, k, v, D ** -0.5, causal)
+    qd, kd, vd = dev(q), dev(k)[None], dev(v)[None]
+    o = torch.empty_like(qd)
+    K.decode_attn(qd, kd, vd, o=o, ctx_len=Skv, causal_off=Skv - Sq if causal else -1, q_strides=(D, Sq * D),
+                  kv_strides=(0, Skv * D), B=Sq, Hq=H)
+    fine = np.isfinite(want)
+    for out, name in ((got, "sdpa"), (host(o), "decode")):
+        np.testing.assert_array_equal(out[~fine].astype(np.float64), want[~fine], err_msg=name)
+        assert (np.abs(out[fine] - want[fine]) <= np.abs(want[fine]) * 2.0 ** -11 + 5 * 2.0 ** -12).all(), name
+
+
 def test_bad_arguments_raise():
     from aneforge_amd import _kernels as K
     t = torch.zeros((2, 16, 32), dtype=torch.float16, device="cuda")
