@@ -491,15 +491,16 @@ class _Lowering:
     def _sdpa_on_mfma(H, Sq, Skv, D):
         """Whether unmasked attention runs on the MFMA kernel (afx_sdpa) rather than the decode kernel, by
         their predicted microseconds.  The decode kernel streams every key for every query (8 M
-        multiply-adds a microsecond: 32 heads x 512 x 512 x 128 measured 129); the MFMA kernel walks
-        64-key blocks, two halves at once, per 64 queries of a head, one workgroup a CU (2.85 us a block at
-        D = 128, 2.0 at 64: the same shape 17).  Few queries over many keys stay on the split-KV kernel."""
+        multiply-adds a microsecond: 32 heads x 512 x 512 x 128 takes 130); the MFMA kernel walks 64-key
+        blocks, two halves at once, per 64 queries of a head, one workgroup a CU (3.2 us a pair of blocks
+        at D = 128, 2.36 at 64: the same shape 18).  Few queries over many keys stay on the split-KV kernel
+        (32 heads x 64 x 2048 x 64 takes 37.5 us there, 40.7 here)."""
         if D not in (64, 128):
             return False
-        blocks = -(-(-(-Skv // 64)) // 2)
+        pairs = -(-(-(-Skv // 64)) // 2)
         rounds = -(-(H * -(-Sq // 64)) // 256)
-        base, block = (4.0, 2.85) if D == 128 else (3.4, 2.0)
-        return base + block * blocks * rounds < 5.0 + H * Sq * Skv * D / 8e6
+        base, pair = (3.6, 3.2) if D == 128 else (2.8, 2.36)
+        return base + pair * pairs * rounds < 5.0 + H * Sq * Skv * D / 8e6
 
     def _op_sdpa(self, t):
         q, k, v = (self.buf[id(s)] for s in t.srcs[:3])

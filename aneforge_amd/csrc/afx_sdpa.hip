@@ -2,13 +2,14 @@
 // shapes, aneforge/graph.py:993-1040), plain or causal, fp32 scores and softmax.
 //
 // The decode kernel takes one query a row and streams the keys through VALU dot products: 512 queries of
-// 32 heads read every key 512 times (137 us, 14 TFLOP/s).  Here both products run on MFMA with keys
-// staged once per 64 queries:
+// 32 heads (8 kv, head dim 128) read every key 512 times (130 us).  Here both products run on
+// MFMA with keys staged once per 64 queries (18 us, causal or not):
 //  * S^T = K Q^T (keys are the A rows): a query's scores sit in four lanes, so row maxima and sums are
 //    lane-local but for two exchanges, and the probabilities are already the B operand of O^T = V^T P^T.
-//  * The probabilities keep 22 bits: p = hi + lo, two fp16 values, each multiplied with V (one third
-//    more products than with p rounded to fp16; no less precise than the decode kernel's fp32 p).  p is
-//    scaled by 2^14 (the sum with it), so lo stays a normal fp16 number.
+//  * The probabilities keep their fp32 bits: p = the sum of three fp16 values, each multiplied with V, so
+//    a product has the decode kernel's fp32 weight; with two (22 bits) differences of near weights came out
+//    ten times further from 64 bits, for 16.2 us instead of 17.7.  The three hold p * 2^14, exactly down to
+//    p = 2^-14 and to 2^-39 below; the power of two leaves with the sum's reciprocal.
 //  * Eight wavefronts: 64 queries x two halves of the keys, each half with its own double-buffered
 //    stages, merged through LDS, so the longest serial chain is half the key blocks (causal tiles are
 //    dispatched longest first).
@@ -17,13 +18,12 @@
 // weight into NaN, and the infinity of a visible one too (its weight's low part may be zero or negative),
 // so a block that holds one adds its visible keys one by one, each with its fp32 weight.  Looking for them
 // takes three VALU operations per two values as they are staged.
-// 32 heads (8 kv) x 512 x 128 causal: 152 -> 22 us.
 #include "afx_common.h"
 
 namespace afx {
 
 constexpr int kSQ = 64, kSB = 64;        // queries per workgroup, keys per block
-constexpr float kPScale = 14.0f;         // log2 of the probabilities' scale
+constexpr float kPScale = 16384.0f;      // the probabilities' scale: the largest is 1, and 2^14 an fp16 number
 
 struct SdpaArgs {
   const half_t *q, *k, *v;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          st[j][e] = __builtin_amdgcn_exp2f(st[j][e] - me + kPScale);
+          st[j][e] = __builtin_amdgcn_exp2f(st[j][e] - me);
           rs += st[j][e];
         }
       lrow = lrow * alpha + swap32_sum(swap16_sum(rs));
@@ -152,14 +152,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           for (int e = 0; e < 4; ++e) acc[d][e] *= alpha;
       }
       if (!odd[hf][i & 3]) {
-        h8 hi[2], lo[2];
+        h8 pf[2][3];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float p = st[2 * ks + (e >> 2)][e & 3];
-            hi[ks][e] = (half_t)p;
-            lo[ks][e] = (half_t)(p - (float)hi[ks][e]);
+            float p = st[2 * ks + (e >> 2)][e & 3] * kPScale;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              pf[ks][i][e] = (half_t)p;
+              p -= (float)pf[ks][i][e];                // exact
+            }
           }
 #pragma unroll
         for (int d = 0; d < ND; ++d)
@@ -172,8 +175,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const v4s a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)vp);
             const v4s a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(vp + 16 * VR));
             const h8 vf = __builtin_bit_cast(h8, (v8s){a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
-            acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, lo[ks], acc[d], 0, 0, 0);
-            acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, hi[ks], acc[d], 0, 0, 0);
+#pragma unroll
+            for (int i = 2; i >= 0; --i) acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[ks][i], acc[d], 0, 0, 0);
           }
       } else {
         // key by key: the weight from the lane that holds it, only where the query sees the key
@@ -185,7 +188,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (j * 4 + e == (key >> 4) * 4 + (key & 3)) p = st[j][e];
-          p = __shfl(p, fr + 16 * ((key >> 2) & 3), 64);
+          p = __shfl(p, fr + 16 * ((key >> 2) & 3), 64) * kPScale;
           if (key0 + key < seen) {
 #pragma unroll
             for (int d = 0; d < ND; ++d) {
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float mn = fmaxf(mrow, mb);
   const float sa = mrow == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mrow - mn);
   const float sb = mb == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mb - mn);
-  const float inv = 1.0f / (lrow * sa + lb * sb);
+  const float inv = 1.0f / (lrow * sa + lb * sb) * (1.0f / kPScale);
   half_t* orow = a.o + ((size_t)h * a.Sq + mq) * D + 4 * fg;
 #pragma unroll
   for (int d = 0; d < ND; ++d) {

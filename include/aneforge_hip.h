@@ -155,7 +155,7 @@ int afx_decode_attn_noalloc(const void* q, const void* k, const void* v, void* o
 
 /* af.sdpa over many queries (aneforge/graph.py:993-1040): o = softmax(q k^T * scale) v for contiguous fp16
  * q / o [H][Sq][D], k / v [Hkv][Skv][D], D 64 or 128, query head h on kv head h / (H / Hkv); causal: query i
- * sees keys 0 .. Skv - Sq + i (Skv >= Sq).  On MFMA with the probabilities kept to 22 bits. */
+ * sees keys 0 .. Skv - Sq + i (Skv >= Sq).  On MFMA with the probabilities' fp32 bits kept. */
 int afx_sdpa(const void* q, const void* k, const void* v, void* o, int H, int Hkv, int Sq, int Skv, int D, int causal,
              float scale, void* stream);
 

@@ -63,6 +63,31 @@ def test_no_less_precise_than_the_decode_kernel(causal):
     assert err[0] <= 1.01 * err[1]                          # both at the fp16 output's rounding
 
 
+@pytest.mark.parametrize("D,Skv", [(64, 64), (128, 64), (128, 49)])
+def test_weights_keep_their_fp32_bits(D, Skv):
+    """Differences of nearly equal weights: a dimension adds one key's weight times 2^15 and takes off the
+    next one's.  Scores are single fp16 products and the largest is 0, and the products and differences are
+    exact, so what is off is the fp32 weights' own last places (a hundred of them make a difference): as far
+    as the decode kernel's, up to how those happen to round.  Weights of 22 bits are off by ten times that."""
+    from aneforge_amd import _kernels as K
+    Sq = 70
+    say(f"sdpa weight bits D={D} Skv={Skv}")
+    rng = np.random.default_rng(D + Skv)
+    q, k, v = np.zeros((1, Sq, D), np.float16), np.zeros((1, Skv, D), np.float16), np.zeros((1, Skv, D), np.float16)
+    q[0, :, 0] = rng.uniform(0.5, 2.0, Sq)
+    for j in range((Skv - 1) // 2):
+        a = np.float16(-rng.uniform(2.0 ** -8, 2.0 ** -5))
+        k[0, 2 * j, 0], k[0, 2 * j + 1, 0] = a, np.nextafter(a, np.float16(0))
+        v[0, 2 * j, j], v[0, 2 * j + 1, j] = 2.0 ** 15, -2.0 ** 15
+    got = _run(q, k, v, 0.37, False).astype(np.float64)
+    qd, kd, vd = dev(q), dev(k)[None], dev(v)[None]
+    o = torch.empty_like(qd)
+    K.decode_attn(qd, kd, vd, o=o, ctx_len=Skv, scale=0.37, q_strides=(D, Sq * D), kv_strides=(0, Skv * D), B=Sq, Hq=1)
+    want = _want(q, k, v, 0.37, False)
+    err = [np.linalg.norm(x.astype(np.float64) - want) / np.linalg.norm(want) for x in (got, host(o))]
+    assert err[0] <= 1.5 * err[1], err
+
+
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 def test_values_hidden_by_the_causal_mask_do_not_leak(bad):
     H, S, D = 2, 150, 64
