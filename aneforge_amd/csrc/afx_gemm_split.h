@@ -501,15 +501,17 @@ extern template split_fn pick_split<FMT_L4>(int, int);
 extern template split_fn pick_split<FMT_Q4K>(int, int);
 extern template split_fn pick_split<FMT_Q6K>(int, int);
 
-// Row tiles (16 * mt rows each), features per tile (32 * nw) and K slices of a dense [M][K] x [N][K] product.
+// Row tiles (16 * mt rows each), features per tile (32 * nw) and K slices of a dense [M][K] x [N][K] product,
+// as many slices as a workspace of ws_bytes holds.
 struct SplitPlan {
   int mt, nw, tiles_m, tiles_n, S;
   float us;                // its predicted time
 };
 bool split_supported(int fmt, int N, int K);
-// afx_gemm_split's launches, `a` filled in but for the plan's fields; w, x and ws 16-byte aligned.
-int split_launch(int fmt, SplitArgs& a, long long ws_bytes, hipStream_t stream, const char* what);
-SplitPlan split_plan(int fmt, int M, int N, int K);
+// afx_gemm_split's launches by plan p (made for a.ws), `a` filled in but for the plan's fields; w, x and ws
+// 16-byte aligned.
+int split_launch(int fmt, SplitArgs& a, const SplitPlan& p, hipStream_t stream, const char* what);
+SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes = 1ll << 62);
 // The grouped experts (a.cnt set): a's pointers, strides, T, E, topk, N, K and epi filled in by the caller.
 int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what);
 

@@ -44,6 +44,10 @@ static float split_chunk_us(int fmt, int mt, int nw, bool busy) {
   const float slow = !busy ? 1.0f : mt == 8 && !alone ? 1.2f : nw == 8 ? 1.2f : 1.0f;
   return nw == 8 ? (c8[i] + 2.0f * dec[fmt]) * slow : (c4[i] + dec[fmt]) * slow * (nw == 4 ? 1.0f : 0.7f);
 }
+static int split_rows_kept(int M) { return M < 16 ? M : 16; }
+static long long split_ws_bytes(const SplitPlan& p, int M, int S) {
+  return (long long)S * p.tiles_m * p.tiles_n * p.mt * p.nw * 128 * split_rows_kept(M);
+}
 static double weight_mb(int fmt, int N, int K) {
   return (double)N * (split_row_bytes_of(fmt, K) + split_side_bytes_of(fmt, K)) * 1e-6;
 }
@@ -54,7 +58,7 @@ static double weight_mb(int fmt, int N, int K) {
 // per MB of partials when K is sliced.  Predictions are within 15% of what the shapes above measure at
 // 16 to 2048 rows: 4096 x 4096 at 64, 128 and 300 rows takes 13.6, 15.9 and 25.2 us where the 128 x 128
 // tiles of afx_gemm take 42.4, 42.5 and 43.7.
-SplitPlan split_plan(int fmt, int M, int N, int K) {
+SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes) {
   static const int mts[6] = {1, 2, 3, 4, 6, 8};
   const char* es = getenv("AFX_GEMM_SPLIT");       // "S", "S.nw" or "S.nw.mt": a fixed choice (tests, tuning), read per call
   int fs = 0, fn = 0, fm = 0;
@@ -71,8 +75,11 @@ SplitPlan split_plan(int fmt, int M, int N, int K) {
       SplitPlan p = {mt, nw, (t16 + mt - 1) / mt, (N + 32 * nw - 1) / (32 * nw), 1, 0.0f};
       const double part = (double)p.tiles_m * p.tiles_n * mt * nw * 2048e-6;   // MB of one slice's partials
       const bool two = split_two_per_cu(fmt, mt, nw);
-      for (int S = 1; S <= kSplitMaxS && S <= nk; ++S) {
-        if (fs ? S != (fs < nk ? fs : nk) : S > 1 && nk / S < 2) continue;
+      int smax = nk < kSplitMaxS ? nk : kSplitMaxS;
+      while (smax > 1 && split_ws_bytes(p, M, smax) > ws_bytes) --smax;
+      if (fs && fs < smax) smax = fs;
+      for (int S = fs ? smax : 1; S <= smax; ++S) {
+        if (!fs && S > 1 && nk / S < 2) continue;
         const double wgs = (double)p.tiles_m * p.tiles_n * S;
         const double rounds = wgs <= 256 ? 1.0 : two ? wgs / 256 + 0.25 : ceil(wgs / 256);
         // a tile's epilogue (its K groups meet, then the stores) grows with its registers
@@ -101,10 +108,6 @@ static float gemm_tile_us(int fmt, int M, int N, int K) {
     us += 2.0 + (2e-6 * N * K + weight_mb(fmt, N, K)) / tbs;
   }
   return (float)us;
-}
-static int split_rows_kept(int M) { return M < 16 ? M : 16; }
-static long long split_ws_bytes(const SplitPlan& p, int M, int S) {
-  return (long long)S * p.tiles_m * p.tiles_n * p.mt * p.nw * 128 * split_rows_kept(M);
 }
 
 // y = epilogue(sum of the S slices of ws in slice order), four output features of one row per thread;
@@ -180,10 +183,8 @@ int split_moe_launch(int fmt, SplitArgs& a, hipStream_t stream, const char* what
   return check_launch(what);
 }
 
-int split_launch(int fmt, SplitArgs& a, long long ws_bytes, hipStream_t stream, const char* what) {
-  const SplitPlan p = split_plan(fmt, a.M, a.N, a.K);
+int split_launch(int fmt, SplitArgs& a, const SplitPlan& p, hipStream_t stream, const char* what) {
   a.S = p.S;
-  while (a.S > 1 && (!a.ws || split_ws_bytes(p, a.M, a.S) > ws_bytes)) --a.S;
   a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.mt = p.mt; a.nw = p.nw;
   a.rp = split_rows_kept(a.M);
   const bool glu = a.epi == EPI_SWIGLU || a.epi == EPI_GEGLU;
@@ -242,7 +243,7 @@ int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int
   a.w = w; a.scale = (const half_t*)scale; a.bias = (const half_t*)bias; a.x = (const half_t*)x; a.y = y;
   a.resid = (const half_t*)residual; a.ldx = ldx; a.ldy = ldy; a.M = M; a.N = N; a.K = K; a.epi = epi;
   a.ws = (float*)ws;
-  return split_launch(fmt, a, ws_bytes, (hipStream_t)stream, "afx_gemm_split");
+  return split_launch(fmt, a, split_plan(fmt, M, N, K, ws ? ws_bytes : 0), (hipStream_t)stream, "afx_gemm_split");
 }
 
 }  // extern "C"

@@ -61,6 +61,33 @@ static int choose_rows(int hint, bool paired, bool norm) {
 // Grid: one row group per wavefront, four wavefronts per workgroup.
 static int grid_for(int ngroups) { return (ngroups + 3) / 4; }
 
+// Predicted microseconds of the kernels that the split GEMM stands in for at few rows, each below what it
+// measures (the lower edge over formats and shapes), so that a call only moves where it gains.
+//
+// The vector kernels (int4 codebook, K-quants): groups of 8 rows, then what is left; a workgroup streams four
+// weight rows, w workgroups a CU (the second comes with the first 16 rows past 1024).  8, 4 and 1 rows of
+// 4096 x 4096 take 30, 11.7 and 4.6 us, of 4096 x 11008 52, 26 and 9, of 22016 x 4096 158, 48 and 15, of
+// 1024 x 4096 8.8, 5.2 and 2.6 (the single rows as a further launch).
+static double vector_us(int M, int N, int K) {
+  const double w = N / 1024.0, k = K / 1000.0;
+  const double us8 = 4.5 + (w <= 1.0 ? 0.9 + 0.66 * k : (w < 2.0 ? 2.0 : w) * (1.5 + 0.97 * k));
+  const double us4 = 3.4 + (w < 1.0 ? 1.0 : w) * 0.48 * k, us1 = 2.4 + (w < 1.0 ? 1.0 : w) * 0.14 * k;
+  const int r = M % 8;
+  return M / 8 * us8 + (r == 0 ? 0.0 : r <= 2 ? us1 : r <= 4 ? us4 : us8);
+}
+// fp16 rows past 4096: the vector kernel below the MFMA kernel's rows (3 rows of 4096 x 11008 26 us, of 22016
+// x 8192 87); its K slices where the workspace holds them and K <= 8192 (8192 x 8192 27 us, 22016 x 4352 37
+// to 43 at 4 to 16 rows); else its tiles, by rounds of workgroups (4096 x 4352 12 us, 8192 x 8192 35, 4096 x
+// 11008 33, 22016 x 11008 153; 100 rows of 4096 x 8192 105).
+static double fp16_rows_us(int M, int N, int K, bool mfma, long long ws_bytes) {
+  const double mb = 2e-6 * N * K;
+  if (!mfma) return 3.5 + 0.215 * mb;
+  const int slices = (K + 1023) / 1024;
+  if (M <= 16 && slices <= 8 && 4LL * slices * M * N <= ws_bytes) return 5.5 + mb / 5.8;
+  const double rounds = (double)((N + 15) / 16) * ((M + 15) / 16) / 256;
+  return 3.0 + (K <= 6144 ? 8.6 : K <= 8192 ? 12.7 : 0.0023 * K) * (rounds < 0.6 ? 0.6 : rounds);
+}
+
 static int launch(int fmt, GemvArgs& a, int eg, int rows_hint, hipStream_t stream, const char* what) {
   AFX_REQUIRE(a.w && a.x && a.y, "%s: null pointer argument", what);
   AFX_REQUIRE(a.M >= 1, "%s: M=%d must be >= 1", what, a.M);
@@ -90,18 +117,28 @@ static int launch(int fmt, GemvArgs& a, int eg, int rows_hint, hipStream_t strea
                     a.vcache,
                 "%s: bad fused-QKV arguments", what);
   // The int4 codebook and the K-quants have no skinny MFMA kernel, and fp16 rows past 4096 leave that
-  // kernel's registers: the split GEMM (afx_gemm_split.h) takes them, with the caller's workspace for
-  // its K slices.  From 5 rows, where the vector kernels take 8 (Q4_K 22016 x 4096 at 8 rows 157 -> 33
-  // us, 2048 x 2048 12 -> 8.4), and from 3 on large matrices (46.6 -> 33; 4096 x 4096 is even there).
+  // kernel's registers: the split GEMM (afx_gemm_split.h) takes them where its plan for the caller's workspace
+  // is the faster, with 10 to 12% for the plans that come out optimistic (several slices, or 128 features
+  // at once).  None of 2100 measured calls at 3 to 200 rows, with and without a workspace, is slower by more
+  // than its runs differ than on the kernel it leaves.  Q4_K 22016 x 4096 at 8 rows 158 -> 33 us, 4096 x 11008 52 -> 21 with a workspace
+  // (without one 47, and 1024 x 4096 stays at 8.8); fp16 4096 x 11008 33 -> 24 with one (stays without: 38).
   const long long weights = (long long)a.N * a.K;
   const bool split_fmt = fmt == FMT_L4 || fmt == FMT_Q4K || fmt == FMT_Q6K || (fmt == FMT_F16 && a.K > 4096);
   if (split_fmt && mfma_min_rows() <= 4 && eg != EG_QKV && !a.gamma && a.M >= (fmt == FMT_F16 || weights >= 40000000 ? 3 : 5) &&
       split_supported(fmt, a.N, a.K) && (!a.ws || ((uintptr_t)a.ws & 15) == 0) &&
       ((long long)(a.M - 1) * a.ldx + a.K) * 2 < (1ll << 31)) {
-    SplitArgs s = {};
-    s.w = a.w; s.scale = a.scale; s.x = a.x; s.ldx = a.ldx; s.y = a.y; s.ldy = a.ldy; s.bias = a.bias; s.resid = a.resid;
-    s.ws = a.ws; s.M = a.M; s.N = a.N; s.K = a.K; s.epi = a.epi;
-    return split_launch(fmt, s, a.ws_bytes, stream, what);
+    const long long ws_bytes = a.ws ? a.ws_bytes : 0;
+    const SplitPlan p = split_plan(fmt, a.M, a.N, a.K, ws_bytes);
+    const bool mfma = fmt == FMT_F16 && a.M >= mfma_min_rows();
+    const bool past = mfma && (2 * weights + 65536 >= 0x7fff0000LL || 2LL * a.M * a.ldx >= 0x7fff0000LL);   // mfma_launch's 2 GiB
+    const double other = fmt == FMT_F16 ? fp16_rows_us(a.M, a.N, a.K, mfma, eg == EG_PLAIN ? ws_bytes : 0)
+                                        : vector_us(a.M, a.N, a.K);
+    if (past || p.us * (p.S > 1 ? 1.12 : p.nw == 4 ? 1.1 : 1.0) < other) {
+      SplitArgs s = {};
+      s.w = a.w; s.scale = a.scale; s.x = a.x; s.ldx = a.ldx; s.y = a.y; s.ldy = a.ldy; s.bias = a.bias; s.resid = a.resid;
+      s.ws = a.ws; s.M = a.M; s.N = a.N; s.K = a.K; s.epi = a.epi;
+      return split_launch(fmt, s, p, stream, what);
+    }
   }
   // 4+ activation rows without a norm prologue: the dot products go to MFMA (any row count, in groups of
   // 16); the vector kernels below take at most 8 rows.  3 rows too on packed matrices of 8 M weights or

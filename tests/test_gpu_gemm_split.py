@@ -341,3 +341,35 @@ def test_planned_tiles(K, fmt, M, N, Kd):
     y = torch.empty((M, N), dtype=torch.float16, device="cuda")
     K.gemm_split(fmt, w, s, dev(x), y, ws=torch.empty(n // 4, dtype=torch.float32, device="cuda") if n else None)
     assert (np.abs(host(y) - want) <= _bound(x, W, want)).all()
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd", [("fp16", 8, 4096, 11008), ("fp16", 16, 512, 5120), ("fp16", 3, 2048, 5632),
+                                        ("q4_k", 8, 1024, 4096), ("lut4", 5, 512, 5120), ("q6_k", 11, 256, 2048)])
+def test_few_rows_without_a_workspace_keep_the_faster_kernel(K, fmt, M, N, Kd):
+    """Without a workspace K is not cut, and these rows are faster on the kernels that take any N: the same
+    bytes as the first N - 4 features by themselves, which only those kernels take."""
+    rng = np.random.default_rng(N + M)
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    say(f"few rows without a workspace {fmt} M={M} N={N} K={Kd}")
+    y = host(K.linear(fmt, w, s, dev(x), out_f32=True))
+    part = host(K.linear(fmt, w[:N - 4], None if s is None else s[:N - 4], dev(x), out_f32=True))
+    want = x.astype(np.float64) @ W.T
+    assert (np.abs(y - want) <= _bound(x, W, want)).all()
+    np.testing.assert_array_equal(y[:, :N - 4], part)
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd,cfg", [("q4_k", 8, 8192, 2048, "1.2.1"), ("lut4", 16, 8192, 2048, "1.2.1"), ("q6_k", 20, 8192, 2048, "1.2.1")])
+def test_few_rows_without_a_workspace_take_an_uncut_tile(K, fmt, M, N, Kd, cfg, monkeypatch):
+    """Where the split GEMM is the faster without a workspace too, it takes the tile that is best uncut (64
+    features), not the one its slices would want: the bytes of that tile."""
+    rng = np.random.default_rng(N + M)
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    say(f"uncut tile {fmt} M={M} N={N} K={Kd}")
+    want = x.astype(np.float64) @ W.T
+    y = host(K.linear(fmt, w, s, dev(x), out_f32=True))
+    assert (np.abs(y - want) <= _bound(x, W, want)).all()
+    monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
+    fixed = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    np.testing.assert_array_equal(y, host(K.gemm_split(fmt, w, s, dev(x), fixed, epi="f32")))
