@@ -144,9 +144,11 @@ static int launch(int fmt, GemvArgs& a, int eg, int rows_hint, hipStream_t strea
   // 16); the vector kernels below take at most 8 rows.  3 rows too on packed matrices of 8 M weights or
   // more whose rows the persistent kernel takes, where the vector kernel's padded fourth row costs more
   // (int8 22016 x 4096 42.5 -> 20 us, Q4_0 4096 x 4096 11.1 -> 6.5; fp16 is even).  Only what mfma_launch
-  // takes: int8 scales on 8 bytes and matrices inside its 2 GiB buffer range; the vector kernel takes the rest.
+  // takes: int8 scales on 8 bytes, and matrices and activations inside its 2 GiB buffer ranges; the vector
+  // kernel takes the rest.
   const bool three = mfma_min_rows() == 4 && weights >= 8000000 && fmt != FMT_F16 && (fmt == FMT_Q4 || a.K <= 4096 || a.ws) &&
-                     ((uintptr_t)a.scale & (fmt == FMT_I8 ? 7 : 3)) == 0 && (fmt == FMT_Q4 ? weights / 2 : weights) + 65536 < 0x7fff0000LL;
+                     ((uintptr_t)a.scale & (fmt == FMT_I8 ? 7 : 3)) == 0 && (fmt == FMT_Q4 ? weights / 2 : weights) + 65536 < 0x7fff0000LL &&
+                     2LL * a.M * a.ldx < 0x7fff0000LL;
   if (a.M >= (three ? 3 : mfma_min_rows()) && eg != EG_QKV && !a.gamma && mfma_supported(fmt, a.K) && a.N % 4 == 0) {
     MfmaArgs m = {};
     m.w = a.w; m.scale = a.scale; m.x = a.x; m.ldx = a.ldx; m.y = a.y; m.ldy = a.ldy;

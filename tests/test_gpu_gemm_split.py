@@ -295,6 +295,21 @@ def test_codebook_rows_past_the_split_range(K):
     assert (np.abs(host(K.linear("lut4", w, s, wide)) - want) <= _bound(x, W, want)).all()
 
 
+@pytest.mark.parametrize("fmt", ["int8", "q4_0", "blockwise"])
+def test_three_rows_that_span_2_gib(K, fmt):
+    """3 rows of a large matrix on a stride of 400 M elements stay on the vector kernel, as 2 rows do."""
+    rng = np.random.default_rng(7)
+    w, s, W = _weights(K, fmt, 2048, 4096, rng)
+    x = rng.standard_normal((3, 4096)).astype(np.float16)
+    wide = torch.empty((3, 400_000_000), dtype=torch.float16, device="cuda")[:, :4096]
+    wide.copy_(dev(x))
+    want = x.astype(np.float64) @ W.T
+    say(f"{fmt} 3 rows, row stride 400M")
+    got = host(K.linear(fmt, w, s, wide))
+    assert (np.abs(got - want) <= _bound(x, W, want)).all()
+    np.testing.assert_array_equal(got[:2], host(K.linear(fmt, w, s, wide[:2])))
+
+
 @pytest.mark.parametrize("slices", [1, 3])
 def test_unused_infinite_codebook_entry(K, slices, monkeypatch):
     """Entry 0 is infinite and no weight names it: the slices' odd last chunks must not bring it in."""
