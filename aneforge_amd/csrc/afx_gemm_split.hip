@@ -14,7 +14,9 @@ static long long split_side_bytes_of(int fmt, int K) {
 }
 
 bool split_supported(int fmt, int N, int K) {
-  return fmt >= 0 && fmt <= 6 && N >= 16 && N % 16 == 0 && K >= kSK && K % (fmt == FMT_Q4K || fmt == FMT_Q6K ? 256 : kSK) == 0;
+  if (fmt < 0 || fmt > 6 || N < 16 || N % 16 != 0 || K < kSK || K % (fmt == FMT_Q4K || fmt == FMT_Q6K ? 256 : kSK) != 0) return false;
+  // a tile's weight rows (up to 256 for the formats with tiles of 256 features) in 31-bit offsets
+  return (fmt == FMT_I8 || fmt == FMT_Q4 ? 256 : 128) * split_row_bytes_of(fmt, K) < (1ll << 31);
 }
 
 // Whether two workgroups share a CU: at most 128 registers a thread and 80 KB of LDS, as the kernels are
@@ -228,7 +230,7 @@ int afx_gemm_split(int fmt, const void* w, const void* scale, const void* x, int
                    void* stream) {
   AFX_REQUIRE(w && x && y, "afx_gemm_split: null pointer");
   AFX_REQUIRE(M >= 1 && split_supported(fmt, N, K),
-              "afx_gemm_split: need M >= 1, N %% 16 == 0, K %% 128 == 0 (256 for K-quants) (fmt=%d M=%d N=%d K=%d)", fmt, M, N, K);
+              "afx_gemm_split: need M >= 1, N %% 16 == 0, K %% 128 == 0 (256 for K-quants), a tile's rows inside 2 GiB (fmt=%d M=%d N=%d K=%d)", fmt, M, N, K);
   AFX_REQUIRE(ldx >= K && ldx % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0,
               "afx_gemm_split: x and weights must be 16-byte aligned rows (ldx %% 8 == 0)");
   AFX_REQUIRE((epi >= 0 && epi <= 3) || epi == EPI_GEGLU, "afx_gemm_split: unknown epilogue %d", epi);

@@ -268,3 +268,11 @@ def test_split_gemm_choice(fmt, M, N, Kd, take):
     """Short prompts on the split GEMM; tall ones, 1 GiB of activations and K below its chunk are not."""
     from aneforge_amd import _kernels as K
     assert K.gemm_split_plan(fmt, M, N, Kd)[0] is take
+
+
+@pytest.mark.parametrize("fmt,N,Kd", [("fp16", 256, 1 << 23), ("int8", 256, 1 << 23), ("q4_0", 256, 1 << 24), ("q4_k", 16, 1 << 25)])
+def test_split_gemm_takes_only_rows_its_offsets_reach(fmt, N, Kd):
+    """A tile's weight rows have to fit 31-bit byte offsets: longer rows are not the split GEMM's."""
+    from aneforge_amd import _kernels as K
+    assert K.gemm_split_plan(fmt, 3, N, Kd) == (False, 0)
+    assert K.gemm_split_plan(fmt, 3, N, Kd - 256)[0]
