@@ -362,7 +362,7 @@ class _Lowering:
         program), as the batched prefill does."""
         M = x2.shape[0]
         if M >= self._GEMM_MIN_ROWS and lin.K % 64 == 0 and lin.N % 16 == 0:
-            split, ws_bytes = E.split_plan(lin, M)
+            split, ws_bytes = E.split_plan(lin, M, x2.stride(0))
             if split:
                 self._ws_bytes = max(self._ws_bytes, ws_bytes)
                 self.steps.append(lambda: K.gemm_split(lin.fmt, lin.w, lin.scale, x2, y2, bias=bias,

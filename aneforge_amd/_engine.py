@@ -242,10 +242,10 @@ def gemm_plan(fmt: str, M: int, N: int, Kd: int):
     return K.gemm_split_plan(fmt, M, N, Kd)
 
 
-def split_plan(lin: "Linear", M: int):
-    """gemm_plan for M rows of lin; weights or scales on odd addresses (views of a caller's own packing)
-    stay on the kernels that take them."""
-    if lin.w.data_ptr() % 16 or (lin.scale is not None and lin.scale.data_ptr() % 16):
+def split_plan(lin: "Linear", M: int, ldx: int = 0):
+    """gemm_plan for M rows, ldx elements apart, of lin; weights or scales on odd addresses (views of a
+    caller's own packing) and rows that span 2 GiB stay on the kernels that take them."""
+    if lin.w.data_ptr() % 16 or (lin.scale is not None and lin.scale.data_ptr() % 16) or M * ldx >= 1 << 30:
         return False, 0
     return gemm_plan(lin.fmt, M, lin.N, lin.K)
 
@@ -262,7 +262,7 @@ def prefill_gemm(eng, lin: "Linear", x, y, residual=None, epi="f16"):
     formats).  Otherwise afx_gemm on the packed weights (int8, fp16), or on the fp16 expansion of the
     others in the engine's weight scratch (for blockwise that measured faster than scaling the codes
     inside the GEMM: 40.7 vs 48.2 ms for the 2048-token cfg3 prompt)."""
-    split, ws_bytes = split_plan(lin, x.shape[0])
+    split, ws_bytes = split_plan(lin, x.shape[0], x.stride(0))
     if split:
         return K.gemm_split(lin.fmt, lin.w, lin.scale, x, y, bias=lin.bias, residual=residual, epi=epi,
                             ws=eng.gemm_scratch(ws_bytes) if ws_bytes else None)

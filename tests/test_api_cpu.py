@@ -276,3 +276,13 @@ def test_split_gemm_takes_only_rows_its_offsets_reach(fmt, N, Kd):
     from aneforge_amd import _kernels as K
     assert K.gemm_split_plan(fmt, 3, N, Kd) == (False, 0)
     assert K.gemm_split_plan(fmt, 3, N, Kd - 256)[0]
+
+
+def test_prompt_rows_that_span_2_gib_leave_the_split_gemm():
+    """A prompt buffer is as wide as the widest layer: its rows may span 2 GiB where they hold far less."""
+    import torch
+    from aneforge_amd import _engine as E
+    raw = torch.zeros(4096 + 16, dtype=torch.uint8)
+    lin = E.Linear("q4_0", raw[-raw.data_ptr() % 16:], None, 4096, 4096)
+    assert E.split_plan(lin, 64)[0] and E.split_plan(lin, 64, (1 << 24) - 8)[0]
+    assert E.split_plan(lin, 64, 1 << 24) == (False, 0)
