@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import os
 from dataclasses import dataclass
 
 import numpy as np
@@ -236,9 +237,10 @@ _GEMM_FMTS = ("int8", "fp16")                    # formats the prefill GEMM read
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_plan(fmt: str, M: int, N: int, Kd: int):
-    """(take the split GEMM, its workspace bytes) for M rows of a packed [N, Kd] weight: a pure function
-    of the shape, so a prompt's launches do not ask the library again."""
+def gemm_plan(fmt: str, M: int, N: int, Kd: int, fixed: str | None = None):
+    """(take the split GEMM, its workspace bytes) for M rows of a packed [N, Kd] weight: a function of the
+    shape and of the override `fixed` that the library reads (AFX_GEMM_SPLIT) alone, so a prompt's linears
+    do not ask again whether to take it; the launch searches its tile for the workspace that it gets."""
     return K.gemm_split_plan(fmt, M, N, Kd)
 
 
@@ -247,7 +249,7 @@ def split_plan(lin: "Linear", M: int, ldx: int = 0):
     caller's own packing) and rows that span 2 GiB stay on the kernels that take them."""
     if lin.w.data_ptr() % 16 or (lin.scale is not None and lin.scale.data_ptr() % 16) or M * ldx >= 1 << 30:
         return False, 0
-    return gemm_plan(lin.fmt, M, lin.N, lin.K)
+    return gemm_plan(lin.fmt, M, lin.N, lin.K, os.environ.get("AFX_GEMM_SPLIT"))
 
 
 @functools.lru_cache(maxsize=4096)

@@ -60,11 +60,9 @@ static double weight_mb(int fmt, int N, int K) {
 // per MB of partials when K is sliced.  Predictions are within 15% of what the shapes above measure at
 // 16 to 2048 rows: 4096 x 4096 at 64, 128 and 300 rows takes 13.6, 15.9 and 25.2 us where the 128 x 128
 // tiles of afx_gemm take 42.4, 42.5 and 43.7.
-SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes) {
+// fs, fn, fm: only these slices (as many of them as fit), features / 32 and rows / 16; 0: any.
+static SplitPlan split_search(int fmt, int M, int N, int K, long long ws_bytes, int fs, int fn, int fm) {
   static const int mts[6] = {1, 2, 3, 4, 6, 8};
-  const char* es = getenv("AFX_GEMM_SPLIT");       // "S", "S.nw" or "S.nw.mt": a fixed choice (tests, tuning), read per call
-  int fs = 0, fn = 0, fm = 0;
-  if (es) sscanf(es, "%d.%d.%d", &fs, &fn, &fm);
   const int nk = K / kSK, t16 = (M + 15) / 16;
   SplitPlan best = {};
   best.us = 1e30f;
@@ -98,6 +96,15 @@ SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes) {
     }
   }
   return best;
+}
+SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes) {
+  const char* es = getenv("AFX_GEMM_SPLIT");       // "S", "S.nw" or "S.nw.mt": a fixed choice (tests, tuning), read per call
+  int fs = 0, fn = 0, fm = 0;
+  if (es && sscanf(es, "%d.%d.%d", &fs, &fn, &fm) >= 1 && fs >= 0 && fn >= 0 && fm >= 0) {
+    const SplitPlan p = split_search(fmt, M, N, K, ws_bytes, fs, fn, fm);
+    if (p.S > 0) return p;                         // else no kernel of that tile is built for the format
+  }
+  return split_search(fmt, M, N, K, ws_bytes, 0, 0, 0);
 }
 // The same product on afx_gemm's 128 x 128 tiles: 0.6 us per 64-wide step with up to a tile per CU, 0.575 us
 // per step and tile of a CU beyond that, after an expansion to fp16 (6 TB/s; the codebook and

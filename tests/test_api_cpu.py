@@ -286,3 +286,28 @@ def test_prompt_rows_that_span_2_gib_leave_the_split_gemm():
     lin = E.Linear("q4_0", raw[-raw.data_ptr() % 16:], None, 4096, 4096)
     assert E.split_plan(lin, 64)[0] and E.split_plan(lin, 64, (1 << 24) - 8)[0]
     assert E.split_plan(lin, 64, 1 << 24) == (False, 0)
+
+
+@pytest.mark.parametrize("fmt,M,cfg", [("lut4", 64, "2.8"), ("int8", 32, "1.8"), ("q4_0", 128, "1.8.8"), ("fp16", 64, "1.2.5"), ("int8", 64, "-1"), ("q4_k", 64, "x")])
+def test_split_gemm_override_that_no_kernel_has(monkeypatch, fmt, M, cfg):
+    """A fixed choice for which no kernel is built leaves the plan as it is."""
+    from aneforge_amd import _kernels as K
+    plan = K.gemm_split_plan(fmt, M, 4096, 4096)
+    assert plan[0]
+    monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
+    assert K.gemm_split_plan(fmt, M, 4096, 4096) == plan
+
+
+def test_cached_split_plan_follows_the_override(monkeypatch):
+    import torch
+    from aneforge_amd import _engine as E
+    raw = torch.zeros(4096 + 16, dtype=torch.uint8)
+    lin = E.Linear("q4_0", raw[-raw.data_ptr() % 16:], None, 4096, 4096)
+    take, nbytes = E.split_plan(lin, 64)
+    assert take and nbytes > 0
+    monkeypatch.setenv("AFX_GEMM_SPLIT", "1.2.4")
+    assert E.split_plan(lin, 64)[1] == 0
+    monkeypatch.setenv("AFX_GEMM_SPLIT", "16.4.4")
+    assert E.split_plan(lin, 64)[1] == 16 * 4096 * 64 * 4
+    monkeypatch.delenv("AFX_GEMM_SPLIT")
+    assert E.split_plan(lin, 64) == (take, nbytes)

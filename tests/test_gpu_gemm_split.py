@@ -388,3 +388,20 @@ def test_few_rows_without_a_workspace_take_an_uncut_tile(K, fmt, M, N, Kd, cfg, 
     monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
     fixed = torch.empty((M, N), dtype=torch.float32, device="cuda")
     np.testing.assert_array_equal(y, host(K.gemm_split(fmt, w, s, dev(x), fixed, epi="f32")))
+
+
+@pytest.mark.parametrize("fmt,M,cfg", [("lut4", 20, "2.8"), ("int8", 20, "1.8"), ("q4_0", 130, "1.8.8"), ("fp16", 20, "1.2.5")])
+def test_override_that_no_kernel_has(K, fmt, M, cfg, monkeypatch):
+    """A fixed choice for which no kernel is built: the plan's own, by its bytes."""
+    rng = np.random.default_rng(M)
+    N, Kd = 272, 512
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    ws = torch.empty(1 << 18, dtype=torch.float32, device="cuda")
+    run = lambda: host(K.gemm_split(fmt, w, s, dev(x), torch.full((M, N), 7.0, dtype=torch.float32, device="cuda"), epi="f32", ws=ws))
+    want = run()
+    exact = x.astype(np.float64) @ W.T
+    assert (np.abs(want - exact) <= _bound(x, W, exact)).all()
+    say(f"override {cfg} {fmt} M={M}")
+    monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
+    np.testing.assert_array_equal(run(), want)
