@@ -10,8 +10,8 @@
 //    meet in LDS at the end, so a tile of 64 features still fills a CU.
 //  * K is cut further into S slices, one workgroup per (tile, slice); the slices' fp32 partials
 //    meet in a caller workspace and a second launch sums them in slice order and applies the
-//    epilogue (S = 1: the epilogue runs here).  Partials cost about 0.5 us per MB, so S is the
-//    smallest count that fills the chip.
+//    epilogue (S = 1: the epilogue runs here).  Partials cost about 0.5 us per MB and the launch 3,
+//    so S and the tile are the ones of least predicted time.
 //  * Global loads are row-contiguous (the MFMA layout would have 16 lanes touch 16 rows: the same
 //    bytes at a quarter of the rate) and run PD chunks ahead in registers; two LDS stages, one
 //    barrier per 128-wide chunk.  Weights are staged in their packed format and decoded when a

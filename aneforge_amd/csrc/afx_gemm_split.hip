@@ -33,18 +33,19 @@ static bool split_two_per_cu(int fmt, int mt, int nw) {
   }
 }
 // Microseconds of one workgroup and K chunk by row tile (16 * mt rows) and features (32 * nw), measured on
-// MI355X with int8 weights at 4096 x 4096 and 22016 x 4096; `busy` with every CU taken, where the taller
-// tiles, one workgroup per CU, slow down (not for the formats whose shorter tiles are alone on a CU too).
+// MI355X; `busy` with every CU taken, where the taller tiles, one workgroup per CU, slow down (not for the
+// formats whose shorter tiles are alone on a CU too).  Tiles of 64 features take 0.7 of 128, taller ones
+// more (their four K groups meet in LDS).
 // dec: what decoding a format's 128 features adds (none for int8 codes, two fp32 steps per weight for the
 // K-quants; fp16: twice the bytes).
 static float split_chunk_us(int fmt, int mt, int nw, bool busy) {
   const int i = mt <= 4 ? mt - 1 : mt <= 6 ? 4 : 5;
-  static const float c4[6] = {0.35f, 0.45f, 0.53f, 0.62f, 0.74f, 0.97f};
-  static const float c8[6] = {0.0f, 0.0f, 0.0f, 1.01f, 1.24f, 1.53f};
+  static const float c4[6] = {0.35f, 0.45f, 0.53f, 0.62f, 0.74f, 0.87f};
+  static const float c8[6] = {0.0f, 0.0f, 0.0f, 1.01f, 1.13f, 1.35f};
   static const float dec[7] = {0.0f, 0.05f, 0.05f, 0.1f, 0.15f, 0.45f, 0.3f};
   const bool alone = fmt == FMT_BW || fmt == FMT_Q4K || fmt == FMT_Q6K;
-  const float slow = !busy ? 1.0f : mt == 8 && !alone ? 1.2f : nw == 8 ? 1.2f : 1.0f;
-  return nw == 8 ? (c8[i] + 2.0f * dec[fmt]) * slow : (c4[i] + dec[fmt]) * slow * (nw == 4 ? 1.0f : 0.7f);
+  const float slow = busy && ((mt == 8 && !alone) || nw == 8) ? 1.08f : 1.0f;
+  return nw == 8 ? (c8[i] + 2.0f * dec[fmt]) * slow : (c4[i] + dec[fmt]) * slow * (nw == 4 ? 1.0f : mt <= 4 ? 0.7f : mt <= 6 ? 0.78f : 0.84f);
 }
 static int split_rows_kept(int M) { return M < 16 ? M : 16; }
 static long long split_ws_bytes(const SplitPlan& p, int M, int S) {
@@ -54,12 +55,16 @@ static double weight_mb(int fmt, int N, int K) {
   return (double)N * (split_row_bytes_of(fmt, K) + split_side_bytes_of(fmt, K)) * 1e-6;
 }
 
-// The tile and slice count with the least predicted time: rounds of workgroups over the CUs (rounds need
-// not be whole where two are resident per CU) x chunks x the chunk time,
-// a round's fill and drain, half of the weight stream's 5 TB/s time (the other half overlaps), and a second launch and about 0.5 us
-// per MB of partials when K is sliced.  Predictions are within 15% of what the shapes above measure at
-// 16 to 2048 rows: 4096 x 4096 at 64, 128 and 300 rows takes 13.6, 15.9 and 25.2 us where the 128 x 128
-// tiles of afx_gemm take 42.4, 42.5 and 43.7.
+// The tile and slice count with the least predicted time: rounds of workgroups over the CUs x chunks x the
+// chunk time, longer by 6% a round up to three (a chip that stays full), a tile's fill and drain, half of the
+// weight stream's 5 TB/s time (the other half overlaps), and a second launch and about 0.5 us per MB of
+// partials when K is sliced.  An XCD takes whole (feature tile, slice) pairs with all their row tiles, so
+// its 32 CUs may get a round more than the chip's average (int8 5120 x 3072 at 1500 rows: 240 workgroups of
+// 256 features, 36 on four of the XCDs, 102 us where 128 features take 63): the rounds are those of the XCD
+// with the most.  Where two workgroups share a CU the second costs 0.85 of a round.  Nine of ten of 2940
+// measured shapes (7 formats, 17 to 2048 rows, K 1024 to 11008) are within 15% of their prediction.
+// 4096 x 4096 at 64, 128 and 300 rows takes 13.9, 16.5 and 24.8 us where the 128 x 128 tiles of afx_gemm
+// take 42.5, 43.5 and 43.6.
 // fs, fn, fm: only these slices (as many of them as fit), features / 32 and rows / 16; 0: any.
 static SplitPlan split_search(int fmt, int M, int N, int K, long long ws_bytes, int fs, int fn, int fm) {
   static const int mts[6] = {1, 2, 3, 4, 6, 8};
@@ -80,13 +85,16 @@ static SplitPlan split_search(int fmt, int M, int N, int K, long long ws_bytes, 
       if (fs && fs < smax) smax = fs;
       for (int S = fs ? smax : 1; S <= smax; ++S) {
         if (!fs && S > 1 && nk / S < 2) continue;
-        const double wgs = (double)p.tiles_m * p.tiles_n * S;
-        const double rounds = wgs <= 256 ? 1.0 : two ? wgs / 256 + 0.25 : ceil(wgs / 256);
+        const double wgs = 8.0 * ((p.tiles_n * S + 7) / 8) * p.tiles_m;   // as if every XCD had the most of them
+        const double n = wgs <= 256 ? 1.0 : ceil(wgs / 256);
+        const double rounds = n > 1.0 && two ? 0.85 * n - 0.1 + 0.15 * (wgs / 256 - (n - 1.0)) : n;
+        const double sustained = 1.0 + 0.06 * (n < 4.0 ? n - 1.0 : 3.0);
+        const double fill = S > 1 ? 0.0 : 0.22 * (mt * nw) * (wgs < 256 ? wgs / 256 : 1.0);
         // a tile's epilogue (its K groups meet, then the stores) grows with its registers
         const double tail = 0.0016 * (mt * nw) * (mt * nw);
-        const double us = 4.5 + rounds * tail + (rounds - 1) * (two ? 1.0 : 2.5) +
-                          rounds * ((nk + S - 1) / S) * split_chunk_us(fmt, mt, nw, wgs > 200) +
-                          weight_mb(fmt, N, K) / 10.0 + (S > 1 ? 2.0 + 0.5 * S * part : 0.0);
+        const double us = 4.5 + rounds * tail + (rounds - 1) * (two ? 1.0 : 2.5) + fill +
+                          sustained * rounds * ((nk + S - 1) / S) * split_chunk_us(fmt, mt, nw, wgs > 200) +
+                          weight_mb(fmt, N, K) / 10.0 + (S > 1 ? 3.0 + 0.5 * S * part : 0.0);
         if (us < best.us) {
           best = p;
           best.S = S;
@@ -106,13 +114,18 @@ SplitPlan split_plan(int fmt, int M, int N, int K, long long ws_bytes) {
   }
   return split_search(fmt, M, N, K, ws_bytes, 0, 0, 0);
 }
-// The same product on afx_gemm's 128 x 128 tiles: 0.6 us per 64-wide step with up to a tile per CU, 0.575 us
-// per step and tile of a CU beyond that, after an expansion to fp16 (6 TB/s; the codebook and
-// K-quant kernels 4 and 2) for formats it does not read.
+// The same product on afx_gemm's tiles, after an expansion to fp16 (6 TB/s; the codebook and K-quant kernels
+// 4 and 2) for formats it does not read.  Microseconds per K step of 64 by the 128 x 128 tiles of a CU on the
+// XCD with the most; fp16's 256 x 256 tiles, where afx_gemm takes them, 1.9 a round.
 static float gemm_tile_us(int fmt, int M, int N, int K) {
-  const double tiles = (double)((M + 127) / 128) * ((N + 127) / 128);
-  double us = 4.5 + (K / 64) * (tiles <= 256 ? 0.6 : 0.575 * tiles / 256 + 0.15) + weight_mb(fmt, N, K) / 12.0;
-  if (fmt != FMT_I8 && fmt != FMT_F16) {
+  const int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+  const double x = 8.0 * ((tiles_n + 7) / 8) * tiles_m / 256, n = ceil(x);
+  const bool i8 = fmt == FMT_I8;
+  double step = n <= 1.0 ? 0.57 + 0.07 * x : n <= 2.0 ? (i8 ? 0.65 : 0.7) + 0.22 * x : (i8 ? 0.52 : 0.55) * n;
+  const double rounds7 = ceil(8.0 * (((N + 255) / 256 + 7) / 8) * ((M + 255) / 256) / 256);
+  if (!i8 && 10.0 * tiles_m * tiles_n >= 34 * 256 * rounds7) step = 1.9 * rounds7;
+  double us = 4.5 + 3.0 * (x < 1.0 ? x : 1.0) + K / 64 * step + weight_mb(fmt, N, K) / 20.0;
+  if (!i8 && fmt != FMT_F16) {
     const double tbs = fmt == FMT_Q6K ? 2.0 : fmt == FMT_Q4K || fmt == FMT_L4 ? 4.0 : 6.0;
     us += 2.0 + (2e-6 * N * K + weight_mb(fmt, N, K)) / tbs;
   }
@@ -225,9 +238,10 @@ int afx_gemm_split_plan(int fmt, int M, int N, int K, long long* ws_bytes) {
   const SplitPlan p = split_plan(fmt, M, N, K);
   if (ws_bytes) *ws_bytes = p.S > 1 ? split_ws_bytes(p, M, p.S) : 0;
   // Up to three of afx_gemm's row tiles the two predictions are taken as they are: int8 22016 x 4096 at 128
-  // rows 51 -> 43 us, 11008 x 2048 at 300 35 -> 26, and no shape more than 3% slower.  Past that the split
-  // kernel's error is the larger (int8 22016 x 4096 at 2048 rows: predicted 0.95 of afx_gemm's time, measured 1.17).
-  const float margin = M <= 384 ? 1.0f : 0.88f;
+  // rows 52 -> 43 us, 11008 x 2048 at 300 34 -> 26.  Past that the two are closer and 5% have to be in it: of
+  // 2940 measured shapes 6 come out more than 3% slower than on the other kernel (9% at most), 96 stay there
+  // that would gain more than 5%.
+  const float margin = M <= 384 ? 1.0f : 0.95f;
   // rows of up to 2 K elements apart stay inside the kernel's 2 GiB activation range
   return (long long)M * K < (1ll << 29) && p.us < margin * gemm_tile_us(fmt, M, N, K) ? 1 : 0;
 }

@@ -311,3 +311,13 @@ def test_cached_split_plan_follows_the_override(monkeypatch):
     assert E.split_plan(lin, 64)[1] == 16 * 4096 * 64 * 4
     monkeypatch.delenv("AFX_GEMM_SPLIT")
     assert E.split_plan(lin, 64) == (take, nbytes)
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd,take", [("int8", 1500, 5120, 3072, False), ("fp16", 1800, 1536, 1024, False), ("fp16", 2048, 1280, 1024, False),
+                                             ("fp16", 1000, 2560, 2048, False), ("q4_k", 1000, 2560, 2048, False), ("fp16", 384, 16384, 3072, False),
+                                             ("q6_k", 1000, 1536, 1024, True), ("blockwise", 1500, 2560, 2048, True)])
+def test_split_gemm_choice_counts_the_busiest_xcd(fmt, M, N, Kd, take):
+    """Products that took 1.1 to 1.7 times as long on the split GEMM with a tile that leaves some XCDs a round
+    more than the others: back on afx_gemm, or (the last two) on a tile that is the faster."""
+    from aneforge_amd import _kernels as K
+    assert K.gemm_split_plan(fmt, M, N, Kd) == (take, 0)
