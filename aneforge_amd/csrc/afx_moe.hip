@@ -643,12 +643,28 @@ static long long fmt_scale_halves(int fmt, long long rows, int K) {
        : fmt == FMT_Q4K ? rows * (K / 256) * 10 : fmt == FMT_Q6K ? rows * (K / 32) * 6 : rows;
 }
 
-// Expert linears on the split GEMM (afx_gemm_split.h): batches of more than 16 tokens, whose weights the
-// skinny kernels would stream once per 16 tokens of an expert, and from 4 tokens the formats without a
-// skinny MFMA kernel.  Pointers and 2 GiB of activations (xrows rows of K) it cannot take stay on the other kernels.
-static bool moe_split_ok(int fmt, int T, long long xrows, int N, int K, const void* w, const void* scale, const void* x) {
+// Where an expert linear of [E][N][K] gains on the split GEMM, against what it leaves (old -> new us):
+//  * The codebook and the K-quants, whose vector kernels stream an expert once per 8 tokens: from 4 tokens on
+//    (Q4_K, 8 experts of 16384 x 2048 at 64 tokens 5.4 times as fast), but for few experts from 8 (9 for rows
+//    past 4096) unless the matrix is wide: 4 tokens over 8 of 2048 x 8192 32 -> 42.
+//  * fp16, whose skinny kernel reaches the memory's rate while an expert has one group of 16 rows: past 14
+//    tokens per expert (20 tokens over 8 of 7168 x 4096 76 -> 100, 100 tokens 1.8 times as fast), or for
+//    long narrow matrices, where that kernel runs one workgroup a CU (8 of 2048 x 8192 at 20 tokens 1.3 times).
+//  * The others, with a skinny MFMA kernel too: past its 16 tokens, unless the matrices are small (8 of 1536 x
+//    1024 at 20 tokens 9.6 -> 10.7).
+static bool moe_split_gains(int fmt, int T, int k, int E, int N, int K) {
+  if (!mfma_supported(fmt, K))
+    return T > 3 && (fmt == FMT_L4 || E >= 16 || N >= 4LL * K || T > (K > 4096 ? 8 : 7));
+  if (T <= 16) return false;
+  const double per = (double)T * k / E;
+  if (fmt == FMT_F16) return per > 14.0 || (K >= 3072 && 4LL * N <= 5LL * K);
+  return K > 1024 || (long long)N * E > 32768 || per > 10.0;
+}
+// ... and takes it: pointers and 2 GiB of activations (xrows rows of K) it cannot take stay on the other kernels.
+static bool moe_split_ok(int fmt, int T, int k, int E, long long xrows, int N, int K, const void* w, const void* scale,
+                         const void* x) {
   const uintptr_t align = fmt == FMT_L4 ? 15 : fmt == FMT_I8 ? 1 : 3;
-  return T > (mfma_supported(fmt, K) ? 16 : 3) && split_supported(fmt, N, K) && w && x && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 &&
+  return moe_split_gains(fmt, T, k, E, N, K) && split_supported(fmt, N, K) && w && x && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 &&
          (fmt == FMT_F16 || (scale && ((uintptr_t)scale & align) == 0)) && xrows * K * 2 < 0x7fff0000LL;
 }
 static int moe_split(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int N, int K,
@@ -748,7 +764,7 @@ int afx_moe_topk(const float* logits, int T, int E, int k, int renorm, float* ga
 // W: [E][2F][D] gate/up interleaved rows (format fmt), x: normed hidden [T][D].
 int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int T, int k, int E, int F, int D,
                    const int* cnt, const int* list, void* act, int rows_hint, void* stream) {
-  if (rows_hint == 0 && moe_split_ok(fmt, T, T, 2 * F, D, w, scale, x))
+  if (rows_hint == 0 && moe_split_ok(fmt, T, k, E, T, 2 * F, D, w, scale, x))
     return moe_split(fmt, w, scale, x, T, k, E, 2 * F, D, cnt, list, act, F, EPI_SWIGLU, (hipStream_t)stream, "afx_moe_gateup");
   if (rows_hint == 0 && mfma_supported(fmt, D) && F % 2 == 0) {
     MfmaArgs m = {};
@@ -772,7 +788,7 @@ int afx_moe_gateup(int fmt, const void* w, const void* scale, const void* x, int
 int afx_moe_down(int fmt, const void* w, const void* scale, const void* act, int T, int k, int E, int F, int D,
                  const int* cnt, const int* list, float* y, int rows_hint, void* ws, long long ws_bytes,
                  void* stream) {
-  if (rows_hint == 0 && moe_split_ok(fmt, T, (long long)T * k, D, F, w, scale, act))
+  if (rows_hint == 0 && moe_split_ok(fmt, T, k, E, (long long)T * k, D, F, w, scale, act))
     return moe_split(fmt, w, scale, act, T, k, E, D, F, cnt, list, y, D, EPI_F32, (hipStream_t)stream, "afx_moe_down");
   if (rows_hint == 0 && mfma_supported(fmt, F) && D % 4 == 0) {
     MfmaArgs m = {};
@@ -836,7 +852,7 @@ int afx_moe_down_combine(int fmt, const void* w, const void* scale, const void* 
                          const void* h, const float* gate, const void* shared, void* out, void* stream) {
   AFX_REQUIRE(h && gate && out && y, "afx_moe_down_combine: null pointer");
   int S = 1;
-  if (mfma_supported(fmt, F) && D % 4 == 0 && !moe_split_ok(fmt, T, (long long)T * k, D, F, w, scale, act)) {
+  if (mfma_supported(fmt, F) && D % 4 == 0 && !moe_split_ok(fmt, T, k, E, (long long)T * k, D, F, w, scale, act)) {
     MfmaArgs m = {};
     m.w = w; m.scale = (const half_t*)scale; m.x = (const half_t*)act; m.ldx = F; m.y = y; m.ldy = D;
     m.cnt = cnt; m.list = list; m.T = T; m.k = k; m.x_by_token = 0; m.N = D; m.K = F; m.epi = EPI_F32;
