@@ -144,10 +144,11 @@ def test_workspace_limits_the_slices_and_bad_shapes_raise(K, monkeypatch):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("E,T,k", [(3, 70, 2), (130, 33, 2), (5, 4, 3)])
+@pytest.mark.parametrize("E,T,k", [(3, 70, 2), (130, 33, 2), (5, 4, 3), (20, 4, 3)])
 def test_grouped_experts(K, fmt, E, T, k):
     """Skewed routing: one expert takes every token (several row tiles), others one row, some none; 130
-    experts need more than one pass over the counts; 4 tokens where the format has no skinny MFMA kernel."""
+    experts need more than one pass over the counts; 4 tokens where the format has no skinny MFMA kernel (the
+    K-quants with the 20 experts only)."""
     rng = np.random.default_rng(E + T)
     D, F = 512, 256
     say(f"grouped experts {fmt} E={E} T={T} k={k}")
@@ -405,3 +406,42 @@ def test_override_that_no_kernel_has(K, fmt, M, cfg, monkeypatch):
     say(f"override {cfg} {fmt} M={M}")
     monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
     np.testing.assert_array_equal(run(), want)
+
+
+def _with_sentinel(K, fmt, w, s, x, W, nbytes, what):
+    """gemm_split with the first nbytes of a larger buffer as its workspace: the result, and nothing written past them."""
+    buf = torch.full((nbytes // 4 + (1 << 21),), 7.0, dtype=torch.float32, device="cuda")
+    n = nbytes // 4
+    say(f"{what} workspace {nbytes}")
+    y = K.gemm_split(fmt, w, s, dev(x), torch.empty((x.shape[0], W.shape[0]), dtype=torch.float16, device="cuda"), ws=buf[:n] if n else None)
+    want = x.astype(np.float64) @ W.T
+    assert (np.abs(host(y) - want) <= _bound(x, W, want)).all(), what
+    assert bool((buf[n:] == 7.0).all()), what
+    return buf[:n]
+
+
+@pytest.mark.parametrize("M", [20, 5])
+def test_slices_stay_inside_the_workspace(K, M, monkeypatch):
+    """Fixed to four slices of 2 x 2 tiles: none, two, three or all of them as the workspace holds them."""
+    rng = np.random.default_rng(M)
+    w, s, W = _weights(K, "int8", 64, 512, rng)
+    x = rng.standard_normal((M, 512)).astype(np.float16)
+    monkeypatch.setenv("AFX_GEMM_SPLIT", "4.2.2")
+    per = 2 * 2 * 128 * min(M, 16)                          # bytes of one slice
+    for nbytes, slices in ((0, 1), (2 * per, 2), (3 * per + 8, 3), (4 * per, 4)):
+        ws = _with_sentinel(K, "int8", w, s, x, W, nbytes, f"M={M} slices={slices}")
+        if slices > 1:                                      # the last slice that fits is written
+            assert bool((ws[(slices - 1) * per // 4:slices * per // 4] != 7.0).any())
+
+
+@pytest.mark.parametrize("fmt,M,N,Kd", [("fp16", 100, 1024, 2816), ("q4_k", 100, 4096, 2816), ("blockwise", 40, 3072, 3072),
+                                        ("q6_k", 5, 4096, 4096), ("int8", 13, 2048, 4096), ("lut4", 16, 4096, 2048), ("q4_0", 64, 4096, 4096)])
+def test_planned_slices_stay_inside_the_planned_workspace(K, fmt, M, N, Kd):
+    """The plan's own slices, with exactly the bytes that it asks for, and with half of them."""
+    rng = np.random.default_rng(M + 1)
+    w, s, W = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    nbytes = K.gemm_split_plan(fmt, M, N, Kd)[1]
+    assert nbytes > 0                                       # a shape whose K is cut
+    _with_sentinel(K, fmt, w, s, x, W, nbytes, f"planned {fmt} M={M}")
+    _with_sentinel(K, fmt, w, s, x, W, nbytes // 32 * 16, f"half {fmt} M={M}")
