@@ -488,19 +488,22 @@ class _Lowering:
                                                K.stream()))
 
     @staticmethod
-    def _sdpa_on_mfma(H, Sq, Skv, D):
+    def _sdpa_on_mfma(H, Sq, Skv, D, Hkv=None):
         """Whether unmasked attention runs on the MFMA kernel (afx_sdpa) rather than the decode kernel, by
-        their predicted microseconds.  The decode kernel streams every key for every query (8 M
-        multiply-adds a microsecond: 32 heads x 512 x 512 x 128 takes 130); the MFMA kernel walks 64-key
-        blocks, two halves at once, per 64 queries of a head, one workgroup a CU (3.2 us a pair of blocks
-        at D = 128, 2.36 at 64: the same shape 18).  Few queries over many keys stay on the split-KV kernel
-        (32 heads x 64 x 2048 x 64 takes 37.5 us there, 40.7 here)."""
+        their predicted microseconds.  The decode kernel streams every key for every query: 8 M
+        multiply-adds a microsecond at most (32 heads x 512 x 512 x 128 takes 130), a fifth less without
+        head groups and a tenth less at least past a whole number of 64 keys.  The MFMA kernel walks 64-key blocks,
+        two halves at once, per 64 queries of a head, one workgroup a CU (3.2 us a pair of blocks at D = 128,
+        2.36 at 64: the same shape 18).  Few queries over many keys stay on the split-KV kernel (32 heads x
+        64 x 2048 x 64 takes 37.5 us there, 40.7 here).  Of 828 measured shapes none is more than 3% slower
+        than on the decode kernel, and 68 stay there that would gain more than 5%."""
         if D not in (64, 128):
             return False
         pairs = -(-(-(-Skv // 64)) // 2)
         rounds = -(-(H * -(-Sq // 64)) // 256)
-        base, pair = (3.6, 3.2) if D == 128 else (2.8, 2.36)
-        return base + pair * pairs * rounds < 5.0 + H * Sq * Skv * D / 8e6
+        base, pair = (4.2, 3.2) if D == 128 else (3.2, 2.36)
+        decode = (5.0 + H * Sq * Skv * D / 8e6) * (1.2 if H == Hkv else 1.05) * (1.1 if Skv % 64 else 1.0)
+        return base + pair * pairs * rounds < decode
 
     def _op_sdpa(self, t):
         q, k, v = (self.buf[id(s)] for s in t.srcs[:3])
@@ -508,7 +511,7 @@ class _Lowering:
         _, H, Sq, D = t.srcs[0].shape
         _, Hkv, Skv, _ = t.srcs[1].shape
         y = self.out(t)
-        if (mask is None and self._sdpa_on_mfma(H, Sq, Skv, D)
+        if (mask is None and self._sdpa_on_mfma(H, Sq, Skv, D, Hkv)
                 and all(b.is_contiguous() and b.data_ptr() % 16 == 0 for b in (q, k, v, y))):
             qh, kh, vh, yh = q.view(H, Sq, D), k.view(Hkv, Skv, D), v.view(Hkv, Skv, D), y.view(H, Sq, D)
             scale, causal = t.attrs["scale"], bool(t.attrs.get("causal"))

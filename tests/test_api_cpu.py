@@ -321,3 +321,11 @@ def test_split_gemm_choice_counts_the_busiest_xcd(fmt, M, N, Kd, take):
     more than the others: back on afx_gemm, or (the last two) on a tile that is the faster."""
     from aneforge_amd import _kernels as K
     assert K.gemm_split_plan(fmt, M, N, Kd) == (take, 0)
+
+
+@pytest.mark.parametrize("H,Hkv,Sq,Skv,D,mfma", [(2, 2, 777, 777, 128, True), (4, 4, 420, 420, 128, True), (32, 8, 64, 512, 128, True),
+                                                 (32, 8, 64, 2048, 64, False), (2, 2, 96, 96, 128, False), (2, 2, 1, 4096, 64, False)])
+def test_sdpa_kernel_choice_near_the_line(H, Hkv, Sq, Skv, D, mfma):
+    """Shapes where the other kernel takes 1.08 to 3.4 times as long."""
+    from aneforge_amd._compile import _Lowering
+    assert _Lowering._sdpa_on_mfma(H, Sq, Skv, D, Hkv) is mfma
