@@ -237,11 +237,16 @@ _GEMM_FMTS = ("int8", "fp16")                    # formats the prefill GEMM read
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_plan(fmt: str, M: int, N: int, Kd: int, fixed: str | None = None):
+def gemm_plan(fmt: str, M: int, N: int, Kd: int, fixed: bytes | None = None):
     """(take the split GEMM, its workspace bytes) for M rows of a packed [N, Kd] weight: a function of the
     shape and of the override `fixed` that the library reads (AFX_GEMM_SPLIT) alone, so a prompt's linears
     do not ask again whether to take it; the launch searches its tile for the workspace that it gets."""
     return K.gemm_split_plan(fmt, M, N, Kd)
+
+
+# os.environ's own dictionary: a look through os.environ takes 0.7 us, once per linear of a prompt whose small
+# launches take 5
+_environ = os.environ._data
 
 
 def split_plan(lin: "Linear", M: int, ldx: int = 0):
@@ -249,7 +254,7 @@ def split_plan(lin: "Linear", M: int, ldx: int = 0):
     caller's own packing) and rows that span 2 GiB stay on the kernels that take them."""
     if lin.w.data_ptr() % 16 or (lin.scale is not None and lin.scale.data_ptr() % 16) or M * ldx >= 1 << 30:
         return False, 0
-    return gemm_plan(lin.fmt, M, lin.N, lin.K, os.environ.get("AFX_GEMM_SPLIT"))
+    return gemm_plan(lin.fmt, M, lin.N, lin.K, _environ.get(b"AFX_GEMM_SPLIT"))
 
 
 @functools.lru_cache(maxsize=4096)

@@ -69,6 +69,7 @@ static double weight_mb(int fmt, int N, int K) {
 static SplitPlan split_search(int fmt, int M, int N, int K, long long ws_bytes, int fs, int fn, int fm) {
   static const int mts[6] = {1, 2, 3, 4, 6, 8};
   const int nk = K / kSK, t16 = (M + 15) / 16;
+  const double stream = 4.5 + weight_mb(fmt, N, K) / 10.0;
   SplitPlan best = {};
   best.us = 1e30f;
   for (int im = 0; im < 6; ++im) {
@@ -80,21 +81,20 @@ static SplitPlan split_search(int fmt, int M, int N, int K, long long ws_bytes, 
       SplitPlan p = {mt, nw, (t16 + mt - 1) / mt, (N + 32 * nw - 1) / (32 * nw), 1, 0.0f};
       const double part = (double)p.tiles_m * p.tiles_n * mt * nw * 2048e-6;   // MB of one slice's partials
       const bool two = split_two_per_cu(fmt, mt, nw);
+      const double chunk[2] = {split_chunk_us(fmt, mt, nw, false), split_chunk_us(fmt, mt, nw, true)};
+      // a tile's epilogue (its K groups meet, then the stores) grows with its registers
+      const double tail = 0.0016 * (mt * nw) * (mt * nw), idle = two ? 1.0 : 2.5;
       int smax = nk < kSplitMaxS ? nk : kSplitMaxS;
       while (smax > 1 && split_ws_bytes(p, M, smax) > ws_bytes) --smax;
       if (fs && fs < smax) smax = fs;
       for (int S = fs ? smax : 1; S <= smax; ++S) {
-        if (!fs && S > 1 && nk / S < 2) continue;
-        const double wgs = 8.0 * ((p.tiles_n * S + 7) / 8) * p.tiles_m;   // as if every XCD had the most of them
-        const double n = wgs <= 256 ? 1.0 : ceil(wgs / 256);
-        const double rounds = n > 1.0 && two ? 0.85 * n - 0.1 + 0.15 * (wgs / 256 - (n - 1.0)) : n;
-        const double sustained = 1.0 + 0.06 * (n < 4.0 ? n - 1.0 : 3.0);
-        const double fill = S > 1 ? 0.0 : 0.22 * (mt * nw) * (wgs < 256 ? wgs / 256 : 1.0);
-        // a tile's epilogue (its K groups meet, then the stores) grows with its registers
-        const double tail = 0.0016 * (mt * nw) * (mt * nw);
-        const double us = 4.5 + rounds * tail + (rounds - 1) * (two ? 1.0 : 2.5) + fill +
-                          sustained * rounds * ((nk + S - 1) / S) * split_chunk_us(fmt, mt, nw, wgs > 200) +
-                          weight_mb(fmt, N, K) / 10.0 + (S > 1 ? 3.0 + 0.5 * S * part : 0.0);
+        if (!fs && S > 1 && nk < 2 * S) break;
+        const long long wgs = 8LL * ((p.tiles_n * S + 7) / 8) * p.tiles_m;   // as if every XCD had the most of them
+        const int n = wgs <= 256 ? 1 : (int)((wgs + 255) / 256);
+        const double rounds = n > 1 && two ? 0.7 * n + 0.05 + 0.15 * wgs / 256 : n;
+        const double sustained = 1.0 + 0.06 * (n < 4 ? n - 1 : 3);
+        const double us = stream + rounds * tail + (rounds - 1.0) * idle + sustained * rounds * ((nk + S - 1) / S) * chunk[wgs > 200] +
+                          (S > 1 ? 3.0 + 0.5 * S * part : 0.22 * (mt * nw) * (wgs < 256 ? wgs / 256.0 : 1.0));
         if (us < best.us) {
           best = p;
           best.S = S;
