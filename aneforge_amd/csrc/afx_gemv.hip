@@ -118,10 +118,11 @@ static int launch(int fmt, GemvArgs& a, int eg, int rows_hint, hipStream_t strea
                 "%s: bad fused-QKV arguments", what);
   // The int4 codebook and the K-quants have no skinny MFMA kernel, and fp16 rows past 4096 leave that
   // kernel's registers: the split GEMM (afx_gemm_split.h) takes them where its plan for the caller's workspace
-  // is the faster, with 10 to 12% for the plans that come out optimistic (several slices, or 128 features
-  // at once).  None of 2100 measured calls at 3 to 200 rows, with and without a workspace, is slower by more
-  // than its runs differ than on the kernel it leaves.  Q4_K 22016 x 4096 at 8 rows 158 -> 33 us, 4096 x 11008 52 -> 21 with a workspace
-  // (without one 47, and 1024 x 4096 stays at 8.8); fp16 4096 x 11008 33 -> 24 with one (stays without: 38).
+  // is the faster, with 10 to 12% for the plans that come out optimistic (several slices, or 128 features at
+  // once).  Of 2100 measured calls at 3 to 200 rows, with and without a workspace, none is slower than on the
+  // kernel that it leaves by more than its runs differ.  8 rows of Q4_K 22016 x 4096 158 -> 33 us; of 4096 x
+  // 11008 52 -> 21 with a workspace (without one 47, predicted 55: they stay); of 1024 x 4096 they stay at 8.8
+  // (20 on it without a workspace, 9.8 with one); fp16 4096 x 11008 33 -> 24 with one (38 without: stays).
   const long long weights = (long long)a.N * a.K;
   const bool split_fmt = fmt == FMT_L4 || fmt == FMT_Q4K || fmt == FMT_Q6K || (fmt == FMT_F16 && a.K > 4096);
   if (split_fmt && mfma_min_rows() <= 4 && eg != EG_QKV && !a.gamma && a.M >= (fmt == FMT_F16 || weights >= 40000000 ? 3 : 5) &&
