@@ -445,3 +445,26 @@ def test_planned_slices_stay_inside_the_planned_workspace(K, fmt, M, N, Kd):
     assert nbytes > 0                                       # a shape whose K is cut
     _with_sentinel(K, fmt, w, s, x, W, nbytes, f"planned {fmt} M={M}")
     _with_sentinel(K, fmt, w, s, x, W, nbytes // 32 * 16, f"half {fmt} M={M}")
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("cfg", ["1.2.1", "3.4.2"])
+def test_rows_keep_to_themselves(K, fmt, cfg, monkeypatch):
+    """Rows of NaN and infinities, the last one (which rows past the end repeat) among them, leave the bytes of
+    the others as they are."""
+    monkeypatch.setenv("AFX_GEMM_SPLIT", cfg)
+    rng = np.random.default_rng(11)
+    M, N, Kd = 37, 272, 1280
+    w, s, _ = _weights(K, fmt, N, Kd, rng)
+    x = rng.standard_normal((M, Kd)).astype(np.float16)
+    ws = torch.empty(1 << 18, dtype=torch.float32, device="cuda")
+    say(f"rows keep to themselves {fmt} {cfg}")
+    run = lambda a: host(K.gemm_split(fmt, w, s, dev(a), torch.empty((M, N), dtype=torch.float32, device="cuda"), epi="f32", ws=ws))
+    clean = run(x)
+    odd = [3, 16, M - 1]
+    x[3], x[16, 1279], x[M - 1, 5] = np.nan, np.inf, -np.inf
+    got = run(x)
+    rest = np.delete(np.arange(M), odd)
+    np.testing.assert_array_equal(got[rest], clean[rest])
+    assert not np.isfinite(got[odd].astype(np.float64)).all()
+    assert np.isnan(got[3]).all()

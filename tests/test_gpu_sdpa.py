@@ -145,3 +145,26 @@ def test_bad_arguments_raise():
     kv = torch.zeros((2, 16, 64), dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="bad lengths"):
         K.sdpa(q, kv, kv, torch.empty_like(q), 1.0, causal=True)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal,Sq,Skv,key", [(False, 70, 200, 3), (False, 70, 64, 63), (True, 150, 150, 149), (True, 150, 150, 70), (True, 40, 300, 5)])
+def test_nan_scores_reach_the_queries_that_see_them(causal, Sq, Skv, key, D):
+    """A NaN key row (also one that is all a query sees of its half) makes the queries that see it NaN, as in the
+    decode kernel, and no others."""
+    from aneforge_amd import _kernels as K
+    H = 2
+    say(f"sdpa NaN key {key} causal={causal} Sq={Sq} Skv={Skv} D={D}")
+    rng = np.random.default_rng(key)
+    q = rng.standard_normal((H, Sq, D)).astype(np.float16)
+    k, v = (rng.standard_normal((H, Skv, D)).astype(np.float16) for _ in range(2))
+    k[1, key, 7] = np.nan
+    got = _run(q, k, v, D ** -0.5, causal)
+    qd, kd, vd = dev(q), dev(k)[None], dev(v)[None]
+    o = torch.empty_like(qd)
+    K.decode_attn(qd, kd, vd, o=o, ctx_len=Skv, causal_off=Skv - Sq if causal else -1, q_strides=(D, Sq * D),
+                  kv_strides=(0, Skv * D), B=Sq, Hq=H)
+    nan = np.zeros(got.shape, bool)
+    nan[1, max(0, key - (Skv - Sq)) if causal else 0:] = True
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(np.isnan(host(o)), nan)
